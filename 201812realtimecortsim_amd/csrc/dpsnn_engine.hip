@@ -41,6 +41,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "dpsnn_exp.h"
@@ -145,7 +146,7 @@ __device__ inline void wave_sync() {
 constexpr int kWaveLTP = 256;    // STDP kernels: 4 waves per block
 
 // Per-sub-population LIFCA parameters, in this order.
-enum { kTau, kTheta, kH, kTarp, kAlphaC, kTauC, kGC, kInvTau, kInvTauC, kParams };
+enum { kTheta, kH, kTarp, kAlphaC, kGC, kInvTau, kInvTauLo, kInvTauC, kInvTauCLo, kParams };
 
 struct DevNet {
   uint32_t N, NW, RS, nsub, npc, ncols, cap, drive;
@@ -235,19 +236,25 @@ struct PhiloxStream {
   uint64_t ctr;
   double spare;  // second uniform of the last block
   int have;
-  __device__ double next() {
-    if (have) {
-      have = 0;
-      return spare;
-    }
+  // one block: two uniforms in [0, 1)
+  __device__ inline void block(double &first, double &second) {
     uint32_t c[4] = {(uint32_t)ctr, (uint32_t)(ctr >> 32), 0u, 0x44505300u};
     philox4x32(c, k0, k1);
     ++ctr;
     const uint64_t a = ((uint64_t)c[0] << 21) ^ (uint64_t)c[1];
     const uint64_t b = ((uint64_t)c[2] << 21) ^ (uint64_t)c[3];
-    spare = (double)(b & ((1ull << 53) - 1)) * 0x1p-53;
+    first = (double)(a & ((1ull << 53) - 1)) * 0x1p-53;
+    second = (double)(b & ((1ull << 53) - 1)) * 0x1p-53;
+  }
+  __device__ double next() {
+    if (have) {
+      have = 0;
+      return spare;
+    }
+    double first;
+    block(first, spare);
     have = 1;
-    return (double)(a & ((1ull << 53) - 1)) * 0x1p-53;
+    return first;
   }
 };
 
@@ -263,41 +270,67 @@ __device__ inline double div_rn(double a, double b, double y) {
   return fma(fma(-q1, b, a), y, q1);
 }
 
+// a / b, correctly rounded, for a divisor whose significand has an odd part B
+// below 2^50 (every float, so every time constant DPSNN reads), with
+// yh = RN(1/b) and yl = RN(1/b - yh).  a yh + RN(a yl) is within 2^-105 of
+// a / b relative, 2^-52 of an ulp of the quotient, and one fma rounds it.
+// A midpoint m between two doubles is further away: with a = A 2^i, A < 2^53,
+// b = B 2^j, |a / b - m| B is a non-zero multiple of half an ulp (i - j is at
+// least the exponent of that half ulp, or A would need 54 bits; a tie would
+// need A >= 2^53 too), so |a / b - m| >= ulp / (2 B).  Two FMA-unit operations
+// in place of div_rn's five.
+__device__ inline double div_short(double a, double yh, double yl) { return fma(a, yh, a * yl); }
+// The divisor's odd significand part is below 2^50 (see div_short).
+static inline bool short_divisor(double b) {
+  int e;
+  const double m = std::frexp(std::fabs(b), &e);  // m 2^53 is an integer
+  return std::ldexp(m, 50) == std::floor(std::ldexp(m, 50));
+}
+
 // --------------------------------------------------------------------------
 // LIFCADynamic, DPSNN_neuron_sim.c:664-824 (second-order, non-Perseo path).
-// The divisions by Tau and TauC use their reciprocals (div_rn); the results
-// are the IEEE quotients.
+// The divisions by Tau and TauC use their reciprocals (div_short); the
+// results are the IEEE quotients.  expTab: dpsnn_exp's table, in LDS.
 // --------------------------------------------------------------------------
+typedef __attribute__((address_space(3))) double lds_f64;
+typedef __attribute__((address_space(3))) uint64_t lds_u64;
+typedef __attribute__((address_space(3))) int16_t lds_i16;
 struct Lifca {
   double v, c, Tr, Te;
-  double Tau, Theta, H, Tarp, AlphaC, TauC, gC, invTau, invTauC;
-  bool fired;
+  double Theta, H, Tarp, AlphaC, gC, invTau, invTauLo, invTauC, invTauCLo;
+  const lds_u64 *expTab;
+  uint32_t fired;
   // Both of the reference's branches (out of / in the refractory period)
   // decay c by the same expression; the out-of-refractory one also moves v.
   // The lanes of a wave take different branches, so v's update is computed
   // for every lane and kept where the neuron is out of its refractory
   // period: the same operations in the same order, without divergent
   // control flow.  Only the refractory exit (exp) stays a branch; it is rare.
-  __device__ inline void event(double t, double I) {
+  // A lane without an event (on = false) passes t = Tr: no time elapses, so
+  // c is multiplied by one, and v and Te are kept; nothing changes.
+  __device__ inline void event(bool on, double t, double I) {
     double deltaT = t - Tr;
     const double TFLES = t - Te;
-    const bool active = TFLES > Tarp;
+    const bool active = on && TFLES > Tarp;
     if (active && Tr - Te < Tarp) {
-      c *= dpsnn_exp(div_rn(-(deltaT - TFLES + Tarp), TauC, invTauC));
+      c *= dpsnn_exp_with(div_short(-(deltaT - TFLES + Tarp), invTauC, invTauCLo), expTab);
       deltaT = TFLES - Tarp;
     }
     const double dtHalf = deltaT / 2;
-    const double rmHalf = div_rn(dtHalf, Tau, invTau);
-    const double rc = div_rn(deltaT, TauC, invTauC);
+    const double rmHalf = div_short(dtHalf, invTau, invTauLo);
+    const double rc = div_short(deltaT, invTauC, invTauCLo);
     double w = v - v * rmHalf - gC * c * dtHalf;
     w = w - w * rmHalf - gC * c * dtHalf;
     w += I;
+    // (kept here: the compiler would move v's update under a branch on
+    // `active`, apart from c's, and lose what overlaps the two)
+    asm volatile("" : "+v"(w));
     c = c * (1 - rc + rc * rc / 2);
     const bool fire = active && w >= Theta;
     v = fire ? H : (active ? w : v);
     c = fire ? c + AlphaC : c;
     Te = fire ? t : Te;
-    fired = fired || fire;
+    fired = fire ? 1u : fired;
     Tr = t;
   }
 };
@@ -526,38 +559,37 @@ __device__ inline uint64_t lane_mask_lt() {
 }
 
 // External bath of one neuron in step t, one event at a time in time order:
-// head is the next event's time (+inf when none is pending); take() returns
-// its value and moves on.
+// at() is the next event's time (kNoEvent when none is pending); take() returns its
+// value and moves on.
 constexpr double kNoEvent = __builtin_huge_val();
 struct ExtReplayCursor {
   const double *time, *value;
   uint32_t x, xe;
-  double head;
-  __device__ inline void start() { head = x < xe ? time[x] : kNoEvent; }
-  __device__ inline double take() {
-    const double v = value[x++];
-    head = x < xe ? time[x] : kNoEvent;
-    return v;
-  }
+  __device__ inline double at() const { return x < xe ? time[x] : kNoEvent; }
+  __device__ inline double take() { return value[x++]; }
   __device__ inline void finish() {}
 };
 
 // The reference's Poisson bath (DPSNN_neuron_sim.c:604-640, :844-851) from
 // the Philox stream: the first due event is always drawn (do-while), the
 // following ones while fewer than the per-ms cap; past the cap only the
-// lapses are drawn.
+// lapses are drawn.  An event takes one Philox block (its value from the
+// first uniform, the lapse to the next event from the second).
 struct ExtPhiloxCursor {
   double a, inv, nextF;
   const double *lut;
   uint32_t cap, nExt;
   bool onE;
   PhiloxStream R;
-  __device__ inline bool due() const { return onE && a < nextF && (nExt == 0 || nExt < cap); }
-  __device__ inline double at() const { return a; }
+  __device__ inline double at() const {
+    return onE && a < nextF && (nExt == 0 || nExt < cap) ? a : kNoEvent;
+  }
   __device__ inline double take() {
-    const double val = lut[(uint32_t)(R.next() * kLutDepth)];
+    double pick, lapse;
+    R.block(pick, lapse);
+    const double val = lut[(uint32_t)(pick * kLutDepth)];
     ++nExt;
-    const double u = 1.0 - R.next();
+    const double u = 1.0 - lapse;
     a += -logf((float)u) * inv;
     return val;
   }
@@ -571,46 +603,32 @@ struct ExtPhiloxCursor {
   }
 };
 
-constexpr int kQueue = 4;  // Philox bath events per lane drawn ahead of the merge
-typedef __attribute__((address_space(3))) double lds_f64;
-
-// The Philox bath with the step's first events drawn ahead (fill, all lanes
-// of the wave together, before the merge): up to kQueue (time, value) pairs
-// per lane in LDS (qt/qv: the lane's column of [kQueue][64]); events past
-// the queue are drawn from the cursor as they come.  The Philox stream is
-// consumed in the same order either way, so the events are the same.
-struct ExtQueuedCursor {
-  ExtPhiloxCursor xp;
-  lds_f64 *qt, *qv;  // LDS-typed: a generic pointer here compiled to flat loads, which wait on global loads
-  uint32_t qi, qn;
-  double head;  // time of the next due event, or kNoEvent
-  __device__ inline void fill(bool on) {
-    qn = 0;
-    for (;;) {
-      const bool d = on && qn < (uint32_t)kQueue && xp.due();
-      if (!__ballot(d)) break;
-      if (d) {
-        qt[qn * kWave] = xp.at();
-        qv[qn * kWave] = xp.take();
-        ++qn;
-      }
+// The bath with its events drawn ahead of the merge, by all lanes of the
+// wave together, into LDS: up to kQueue (time, value) pairs per lane, then a
+// time of kNoEvent (qt/qv: the lane's columns of [kQueue + 1][64] and
+// [kQueue][64]).  A lane that has taken its last drawn event while another
+// one is due draws the next ones there and then, through LDS as well: the
+// merge loop itself never waits on a global load.  The stream is consumed in
+// the same order either way, so the events are the same.  Whether another
+// event is due after the drawn ones (its time is not kept: the cursor has it).
+constexpr int kQueue = 4;
+template <class Cursor>
+__device__ __attribute__((always_inline)) inline bool draw_bath(Cursor &x, bool on, lds_f64 *qt, lds_f64 *qv) {
+  uint32_t n = 0;
+  double a = on ? x.at() : kNoEvent;
+  for (;;) {
+    const bool d = n < (uint32_t)kQueue && a < kNoEvent;
+    if (!__ballot(d)) break;
+    if (d) {
+      qt[n * kWave] = a;
+      qv[n * kWave] = x.take();
+      a = x.at();
+      ++n;
     }
-    qi = 0;
-    head = qn ? qt[0] : (on && xp.due() ? xp.at() : kNoEvent);
   }
-  __device__ inline double take() {
-    double v;
-    if (qi < qn) {
-      v = qv[qi * kWave];
-      ++qi;
-    } else {
-      v = xp.take();
-    }
-    head = qi < qn ? qt[qi * kWave] : (xp.due() ? xp.at() : kNoEvent);
-    return v;
-  }
-  __device__ inline void finish() { xp.finish(); }
-};
+  qt[n * kWave] = kNoEvent;
+  return a < kNoEvent;
+}
 
 constexpr int kChunk = 8;  // internal events per lane per LDS-staged chunk
 // From step kPackT on, a scratch entry carries its weight in the low 16 bits
@@ -619,16 +637,22 @@ constexpr int kChunk = 8;  // internal events per lane per LDS-staged chunk
 // steps keep the weight in its own array.
 constexpr uint32_t kPackT = 32;
 constexpr int kRun = 16;   // events per neuron run in the blocked scratch
-// LDS of one wave in phase 2: one chunk of 64 lanes' ticks, a row of
-// kStageRow per event (the wave has read all of a chunk before it stores the
-// next one over it), then the bath queue (times, values: [kQueue][64]
-// doubles each).  A row is 64 ticks plus 8 of padding: the transposing
-// stores write 8 rows x 8 neurons per instruction, which a 64-wide row would
-// put on one bank per neuron (8-way conflicts); 72 spreads them over all 64
-// banks.
-constexpr uint32_t kStageRow = kWave + 8;
-constexpr size_t kStageKBytes = kChunk * kStageRow * sizeof(uint64_t);
-constexpr size_t kStageBytes = kStageKBytes + 2 * kQueue * kWave * sizeof(double);
+// LDS of one wave in phase 2: a ring of two chunks of 64 lanes' ticks, a row
+// of kStageRow per event, then the bath queue (values, then times and their
+// end mark: [kQueue][64] and [kQueue + 1][64] doubles) and, for steps before kPackT, the
+// ring's weights.  The lanes
+// move through the ring each at its own pace (a lane that takes bath events
+// falls behind the others): a chunk is stored over the one before the last
+// when every lane is past that.  A row is 64 ticks plus padding: the
+// transposing stores write 8 rows x 8 neurons per instruction, which 64-wide
+// rows would put on one bank per neuron.
+constexpr uint32_t kRing = 2 * kChunk;
+constexpr uint32_t kStageRow = kWave + 1;
+constexpr size_t kStageKBytes = kRing * kStageRow * sizeof(uint64_t);
+constexpr size_t kStagePackedBytes = kStageKBytes + (2 * kQueue + 1) * kWave * sizeof(double);
+constexpr size_t kStageBytes = kStagePackedBytes + kRing * kWave * sizeof(int16_t);
+constexpr uint32_t kExpTab = 256;  // words of dpsnn_exp's table
+constexpr size_t kExpTabBytes = kExpTab * sizeof(uint64_t);
 
 // A buffer view of `bytes` (< 2^31) bytes at base (raw: stride 0, byte
 // offsets; the gfx9 descriptor word).  An access at kDropOffset is out of
@@ -670,53 +694,89 @@ __device__ inline void load_chunk(const __amdgpu_buffer_rsrc_t &tileK, const int
   }
   if (!packed) rw = *(const uint4 *)(tileW + blk + (size_t)lane * kRun);
 }
-__device__ inline void store_chunk(uint64_t *stageK, const uint64_t (&rk)[kChunk]) {
-  const uint32_t lane = threadIdx.x & 63, e = lane & 7;
+// Chunk c into its half of the ring.
+__device__ inline void store_chunk(lds_u64 *ring, lds_i16 *ringW, uint32_t c, const uint64_t (&rk)[kChunk],
+                                   const uint4 &rw, bool packed) {
+  const uint32_t lane = threadIdx.x & 63, e = lane & 7, half = (c & 1) * kChunk;
 #pragma unroll
-  for (int r = 0; r < kChunk; ++r) stageK[e * kStageRow + (uint32_t)r * 8 + (lane >> 3)] = rk[r];
+  for (int r = 0; r < kChunk; ++r) ring[(half + e) * kStageRow + (uint32_t)r * 8 + (lane >> 3)] = rk[r];
+  if (!packed) {
+    const uint32_t w[4] = {rw.x, rw.y, rw.z, rw.w};
+#pragma unroll
+    for (int i = 0; i < kChunk; ++i) ringW[(half + i) * kWave + lane] = (int16_t)(w[i / 2] >> (16 * (i & 1)));
+  }
+}
+
+// dpsnn_exp's table into LDS, by the block's threads (a barrier must follow).
+__device__ inline void load_exp_table(lds_u64 *tab) {
+  for (uint32_t i = threadIdx.x; i < kExpTab; i += blockDim.x) tab[i] = dpsnn_exp_tab_d[i];
 }
 
 // Phase 2, one lane per neuron: lane q integrates neuron j0 + q (q < m) over
 // its n sorted internal events (the tile's blocked scratch tileK/tileW:
 // ticks relative to bits(t) and int16 weights) merged with its external
-// bath, LIFCADynamic per event in FP64.  The events are staged through LDS
-// (stage, kStageBytes) a chunk ahead.  Returns the lane's external event
+// bath, LIFCADynamic per event in FP64.  Returns the lane's external event
 // count and whether (and when) its neuron fired.  Whole wave, uniform.
 // PK 1: every entry carries its weight (t >= kPackT), PK 2: t decides at
-// run time.  The packed-only form needs 16 fewer VGPRs (128: 4 waves/SIMD
-// instead of 3).
+// run time.
+//
+// A neuron's events are one serial chain, so a wave's time is its longest
+// neuron's events times the latency of one turn of the merge loop, and what
+// bounds the kernel is that latency while there are fewer waves than SIMDs
+// (grids up to 8x8 columns) and FP64 issue beyond.  Hence the loop:
+//  * takes nothing from global memory: the events are staged through LDS two
+//    chunks deep with the third in flight, the bath is queued in LDS and
+//    exp's table is there (stage, kStageBytes; expTab).  A load anywhere in
+//    the loop makes the compiler wait for all of them on every turn, the
+//    chunk in flight included;
+//  * lets every lane go on at its own pace through the ring, so that a
+//    wave's turns are the most events of one lane, not the sum over chunks
+//    of the most events in the chunk;
+//  * is one straight block: a lane without an event runs one that changes
+//    nothing; drawing more of the bath and the refractory exit are the only
+//    branches, and rare.
+// Measured, us per launch, before and after: 5,000 neurons 208 -> 145,
+// 80,000 neurons 308 -> 226, 720,000 neurons 1155 -> 964.
 template <bool REPLAY, int PK = 2>
 __device__ __attribute__((always_inline)) inline uint32_t integrate_wave(const DevNet &P, uint32_t t, const ExtView &X, uint32_t j0, uint32_t m,
-                                          const uint64_t *tileK, const int16_t *tileW, uint32_t n, uint8_t *stage,
-                                          bool &fired, double &te) {
+                                          const uint64_t *tileK, const int16_t *tileW, uint32_t n, lds_u64 *stage,
+                                          const lds_u64 *expTab, bool &fired, double &te) {
   const uint32_t lane = threadIdx.x & 63;
   const bool on = lane < m;
   const uint32_t j = j0 + lane;
   if (!on) n = 0;
   uint32_t nmax = n;
   for (int o = 32; o > 0; o >>= 1) nmax = max(nmax, (uint32_t)__shfl_xor((int)nmax, o));
+  nmax = (uint32_t)__builtin_amdgcn_readfirstlane((int)nmax);
   const double tF = (double)t, nextF = (double)(tF + 1.0);
   const uint64_t tBits = dpsnn_asu64(tF);
+  const bool packed = PK == 2 ? t >= kPackT : PK == 1;
+  const __amdgpu_buffer_rsrc_t tileR = buffer_view(wave_uniform(tileK), P.cap * kWave * (uint32_t)sizeof(uint64_t));
+  const uint32_t chunks = (nmax + kChunk - 1) / kChunk;
+  lds_u64 *ring = stage;
+  lds_i16 *ringW = (lds_i16 *)((__attribute__((address_space(3))) uint8_t *)stage + kStagePackedBytes);
+  uint64_t rk[kChunk];
+  uint4 rw = make_uint4(0, 0, 0, 0);
+  if (chunks) load_chunk(tileR, tileW, 0, __ballot(n > 0), rk, rw, packed);
   Lifca L;
   uint32_t sp = 0;
+  L.expTab = expTab;
   if (on) {
     sp = P.subPop[j];
     const double *prm = P.sp + (size_t)sp * kParams;
     L.v = P.v[j]; L.c = P.c[j]; L.Tr = P.Tr[j]; L.Te = P.Te[j];
-    L.Tau = prm[kTau]; L.Theta = prm[kTheta]; L.H = prm[kH]; L.Tarp = prm[kTarp];
-    L.AlphaC = prm[kAlphaC]; L.TauC = prm[kTauC]; L.gC = prm[kGC];
-    L.invTau = prm[kInvTau]; L.invTauC = prm[kInvTauC];
+    L.Theta = prm[kTheta]; L.H = prm[kH]; L.Tarp = prm[kTarp]; L.AlphaC = prm[kAlphaC]; L.gC = prm[kGC];
+    L.invTau = prm[kInvTau]; L.invTauLo = prm[kInvTauLo];
+    L.invTauC = prm[kInvTauC]; L.invTauCLo = prm[kInvTauCLo];
   }
-  L.fired = false;
-  ExtReplayCursor xr{};
-  xr.head = kNoEvent;
-  ExtQueuedCursor xq{};
+  L.fired = 0;
+  std::conditional_t<REPLAY, ExtReplayCursor, ExtPhiloxCursor> bath{};
+  lds_f64 *qv = (lds_f64 *)stage + kRing * kStageRow + lane, *qt = qv + kQueue * kWave;
   if (on) {
-    if (REPLAY) {
-      xr = ExtReplayCursor{X.time, X.value, X.off[j], X.off[j + 1], kNoEvent};
-      xr.start();
+    if constexpr (REPLAY) {
+      bath = ExtReplayCursor{X.time, X.value, X.off[j], X.off[j + 1]};
     } else {
-      ExtPhiloxCursor &xp = xq.xp;
+      ExtPhiloxCursor &xp = bath;
       xp.a = P.assigned[j];
       xp.inv = P.invNuExt[j];
       xp.nextF = nextF;
@@ -727,84 +787,80 @@ __device__ __attribute__((always_inline)) inline uint32_t integrate_wave(const D
       xp.R = PhiloxStream{(uint32_t)P.philoxSeed, (uint32_t)(P.philoxSeed >> 32) ^ j, P.philoxCtr[j], 0.0, 0};
     }
   }
-  if (!REPLAY) {
-    lds_f64 *q = (lds_f64 *)(stage + kStageKBytes);
-    xq.qt = q + lane;
-    xq.qv = q + kQueue * kWave + lane;
-    xq.fill(on);
+  bool due = draw_bath(bath, on, qt, qv);  // a bath event is due after the drawn ones
+  uint32_t qi = 0;                         // the next bath event
+  double head = qt[0], headV = qv[0];
+  if (chunks) store_chunk(ring, ringW, 0, rk, rw, packed);
+  if (chunks > 1) {
+    load_chunk(tileR, tileW, 1, __ballot(n > kChunk), rk, rw, packed);
+    store_chunk(ring, ringW, 1, rk, rw, packed);
   }
-  // one merge loop with a single LIFCADynamic site: internal events from
-  // the staged chunk, the bath event instead when it is strictly earlier
-  // (internal first on equal times), and the rest of the bath once the
-  // lane's internal events are used up
-  const uint32_t chunks = (nmax + kChunk - 1) / kChunk;
-  const uint32_t iters = chunks ? chunks : 1u;
-  uint64_t *stageK = (uint64_t *)stage;  // [kChunk][kStageRow]
-  uint64_t rk[kChunk];
-  uint4 wCur = make_uint4(0, 0, 0, 0), wNext = wCur;
-  const bool packed = PK == 2 ? t >= kPackT : PK == 1;
-  const __amdgpu_buffer_rsrc_t tileR = buffer_view(wave_uniform(tileK), P.cap * kWave * (uint32_t)sizeof(uint64_t));
-  if (chunks) {
-    load_chunk(tileR, tileW, 0, __ballot(n > 0), rk, wCur, packed);
-    store_chunk(stageK, rk);
+  // the loads above are waited for here: one that is still in flight at the
+  // loop's entry would be waited for, with the chunk in flight, on every turn
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  uint32_t staged = min(chunks, 2u);   // chunks stored so far
+  uint32_t e = 0;                     // the lane's next internal event
+  for (;;) {
+    const bool more = staged < chunks;
+    if (more) load_chunk(tileR, tileW, staged, __ballot(n > staged * kChunk), rk, rw, packed);
     wave_sync();
-  }
-  for (uint32_t c = 0; c < iters; ++c) {
-    const uint64_t *curK = stageK;
-    const bool more = c + 1 < chunks;
-    if (more) load_chunk(tileR, tileW, c + 1, __ballot(n > (c + 1) * kChunk), rk, wNext, packed);
-    uint64_t wlo = (uint64_t)wCur.x | ((uint64_t)wCur.y << 32), whi = (uint64_t)wCur.z | ((uint64_t)wCur.w << 32);
-    const uint32_t left = n > c * kChunk ? min((uint32_t)kChunk, n - c * kChunk) : 0u;
-    const bool last = c * kChunk + left >= n;
-    uint32_t e = 0;
-    // the next internal event's entry is read as soon as the previous one is
-    // taken, so that the LDS read overlaps the event's dynamics
-    uint64_t kv = left ? curK[lane] : 0ull;
-    for (;;) {
-      const bool hasI = e < left;
-      const double kI = dpsnn_asf64(tBits + (packed ? kv >> 16 : kv));
-      // the bath event goes first when strictly earlier than the internal
-      // one; with no internal event left in this chunk, only on the last
-      // chunk (otherwise the next chunk is staged first)
-      const double lim = hasI ? kI : (last ? kNoEvent : -kNoEvent);
-      const double hx = REPLAY ? xr.head : xq.head;
-      double at, val;
-      if (hx < lim) {
-        at = hx;
-        val = REPLAY ? xr.take() : xq.take();
-      } else if (hasI) {
-        const int16_t w16 = (int16_t)(uint16_t)(packed ? kv : wlo);
-        wlo = (wlo >> 16) | (whi << 48);
-        whi >>= 16;
-        at = kI;
-        val = (double)(((float)w16) * P.w2f);
-        ++e;
-        if (e < left) kv = curK[e * kStageRow + lane];
-      } else {
-        break;
+    // events of the lane that are staged, those it must be past before the
+    // next chunk is stored, and what a lane without a staged event may take:
+    // any bath event once its internal ones are used up, else none
+    const uint32_t have = min(n, staged * kChunk), need = more ? min(n, (staged - 1) * kChunk) : 0u;
+    const uint64_t final = more ? 0ull : ~0ull;  // the last chunks: on while a lane has an event
+    const double without = n <= staged * kChunk ? kNoEvent : -kNoEvent;
+    // the entry of the next internal event is read as soon as the one before
+    // it is taken, so that the LDS read overlaps the event's dynamics
+    uint64_t kv = ring[(e % kRing) * kStageRow + lane];
+    int16_t kw = packed ? 0 : ringW[(e % kRing) * kWave + lane];
+    // merge: the bath event goes first when strictly earlier
+    bool inner = e < have;
+    double kI = dpsnn_asf64(tBits + (packed ? kv >> 16 : kv));
+    bool outer = head < (inner ? kI : without);
+    const auto go_on = [&] {
+      return (__ballot(e < need) | ((__ballot(inner) | __ballot(outer)) & final)) != 0ull;
+    };
+    if (go_on()) do {
+      const double at = outer ? head : (inner ? kI : L.Tr);
+      const int16_t w16 = packed ? (int16_t)(uint16_t)kv : kw;
+      const double val = outer ? headV : (double)(((float)w16) * P.w2f);
+      const bool some = inner || outer;
+      e += inner && !outer ? 1u : 0u;
+      qi += outer ? 1u : 0u;
+      kv = ring[(e % kRing) * kStageRow + lane];
+      if (!packed) kw = ringW[(e % kRing) * kWave + lane];
+      if (due && qi == (uint32_t)kQueue) {
+        due = draw_bath(bath, true, qt, qv);
+        qi = 0;
       }
-      L.event(at, val);
-    }
-    if (more) {
-      store_chunk(stageK, rk);
-      wCur = wNext;
-    }
+      head = qt[qi * kWave];
+      headV = qv[qi * kWave];
+      L.event(some, at, val);
+      inner = e < have;
+      kI = dpsnn_asf64(tBits + (packed ? kv >> 16 : kv));
+      outer = head < (inner ? kI : without);
+    } while (go_on());
+    if (!more) break;
     wave_sync();
+    store_chunk(ring, ringW, staged, rk, rw, packed);
+    ++staged;
   }
   uint32_t nExt = 0;
   if (on) {
-    if (REPLAY) {
-      nExt = xr.xe - X.off[j];
+    if constexpr (REPLAY) {
+      nExt = bath.xe - X.off[j];
     } else {
-      xq.finish();
-      nExt = xq.xp.nExt;
-      P.assigned[j] = xq.xp.a;
-      P.philoxCtr[j] = xq.xp.R.ctr;
+      bath.finish();
+      nExt = bath.nExt;
+      P.assigned[j] = bath.a;
+      P.philoxCtr[j] = bath.R.ctr;
     }
     P.v[j] = L.v; P.c[j] = L.c; P.Tr[j] = L.Tr; P.Te[j] = L.Te;
   }
-  fired = on && L.fired;
+  fired = on && L.fired != 0;
   te = L.Te;
+  wave_sync();  // the stage is free again
   return nExt;
 }
 
@@ -1182,8 +1238,8 @@ struct NextScan {
 
 // LDS of one wave of the fused step: phase 1's sort, then phase 2's stage.
 __host__ __device__ inline size_t step_lds(uint32_t cap, int B) {
-  const size_t p1 = phase1_lds(cap, B);
-  return p1 > kStageBytes ? p1 : kStageBytes;
+  const size_t p1 = phase1_lds(cap, B), p2 = kStageBytes + kExpTabBytes;
+  return p1 > p2 ? p1 : p2;
 }
 
 // One tile (neurons 64*tile .. 64*tile+63) of step t, one wave: phase 1 for
@@ -1211,12 +1267,15 @@ __device__ __attribute__((always_inline)) inline unsigned long long step_tile(co
   __syncthreads();
   // ---------------- phase 2 ----------------
   const uint32_t n = lane < m ? wcnt[lane] : 0u;
+  lds_u64 *stage = (lds_u64 *)lds, *expTab = stage + kStageBytes / sizeof(uint64_t);
+  load_exp_table(expTab);
+  __syncthreads();
   bool f = false;
   double te = 0.0;
   if (P.drive == DPSNN_DRIVE_REPLAY)
-    exSum += integrate_wave<true>(P, t, X, j0, m, wkeys, wW, n, lds, f, te);
+    exSum += integrate_wave<true>(P, t, X, j0, m, wkeys, wW, n, stage, expTab, f, te);
   else
-    exSum += integrate_wave<false>(P, t, X, j0, m, wkeys, wW, n, lds, f, te);
+    exSum += integrate_wave<false>(P, t, X, j0, m, wkeys, wW, n, stage, expTab, f, te);
   // ---------------- fired scan of step t+1 ----------------
   const uint64_t mask = publish_spikes(P, t + 1, j0 + lane, f, te, S.popCnt, S.count);
   if (S.ltp) ltp_word(P, t + 1, mask, j0);
@@ -1668,12 +1727,21 @@ __global__ __launch_bounds__(kWave) void k_sort_big(DevNet P, uint32_t t) {
   }
 }
 
+// LDS of an integration block: exp's table and each wave's stage.
+template <int PK>
+struct IntegrateLds {
+  uint64_t expTab[kExpTab];
+  uint64_t stage[kBlock / kWave][(PK == 1 ? kStagePackedBytes : kStageBytes) / sizeof(uint64_t)];
+};
+
 // Blocks of kBlock threads: each wave holds 64 consecutive neurons starting
 // at a multiple of 64, as publish_spikes requires.
 template <int PK>
 __global__ __launch_bounds__(kBlock) void k_integrate(DevNet P, uint32_t t, ExtView X, NextScan S) {
-  __shared__ uint8_t stage[kBlock / kWave][kStageBytes];
+  __shared__ IntegrateLds<PK> S2;
   if (P.tDev) t = *P.tDev;
+  load_exp_table((lds_u64 *)S2.expTab);
+  __syncthreads();
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (blockIdx.x == 0 && threadIdx.x < kXcds) P.workCtr[threadIdx.x * kCtrStride] = 0;  // for the next k_gather
   if (blockIdx.x == 0 && threadIdx.x == 0 && P.bigCount) *P.bigCount = 0;                 // for the next k_sort
@@ -1685,9 +1753,11 @@ __global__ __launch_bounds__(kBlock) void k_integrate(DevNet P, uint32_t t, ExtV
   double te = 0.0;
   unsigned long long ex;
   if (P.drive == DPSNN_DRIVE_REPLAY)
-    ex = integrate_wave<true, PK>(P, t, X, j0, m, P.keys + at, P.keyW + at, n, stage[wave], f, te);
+    ex = integrate_wave<true, PK>(P, t, X, j0, m, P.keys + at, P.keyW + at, n, (lds_u64 *)S2.stage[wave],
+                                  (lds_u64 *)S2.expTab, f, te);
   else
-    ex = integrate_wave<false, PK>(P, t, X, j0, m, P.keys + at, P.keyW + at, n, stage[wave], f, te);
+    ex = integrate_wave<false, PK>(P, t, X, j0, m, P.keys + at, P.keyW + at, n, (lds_u64 *)S2.stage[wave],
+                                   (lds_u64 *)S2.expTab, f, te);
   publish_spikes(P, t + 1, j0 + lane, f, te, S.popCnt, S.count);  // LTP follows in k_ltp
   for (int o = 32; o > 0; o >>= 1) ex += __shfl_down(ex, o);
   if (lane == 0 && ex) atomicAdd(counter_slot(P.counters) + 1, ex);
@@ -1746,7 +1816,9 @@ __global__ __launch_bounds__(kBlock) void k_batch_integrate(const DevNet *nets, 
                                                             uint32_t count, uint32_t g0, uint32_t g1, uint32_t cap,
                                                             const uint64_t *keys, const int16_t *keyW,
                                                             const uint32_t *keyCount, uint32_t *workCtr) {
-  __shared__ uint8_t stage[kBlock / kWave][kStageBytes];
+  __shared__ IntegrateLds<PK> S2;
+  load_exp_table((lds_u64 *)S2.expTab);
+  __syncthreads();
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (blockIdx.x == 0 && threadIdx.x < kXcds) workCtr[threadIdx.x * kCtrStride] = 0;  // for the next chunk's gather
   const uint32_t g = g0 + blockIdx.x * (kBlock / kWave) + wave;
@@ -1762,9 +1834,11 @@ __global__ __launch_bounds__(kBlock) void k_batch_integrate(const DevNet *nets, 
   double te = 0.0;
   unsigned long long ex;
   if (P.drive == DPSNN_DRIVE_REPLAY)
-    ex = integrate_wave<true, PK>(P, it.t, it.X, j0, m, keys + at, keyW + at, n, stage[wave], f, te);
+    ex = integrate_wave<true, PK>(P, it.t, it.X, j0, m, keys + at, keyW + at, n, (lds_u64 *)S2.stage[wave],
+                                  (lds_u64 *)S2.expTab, f, te);
   else
-    ex = integrate_wave<false, PK>(P, it.t, it.X, j0, m, keys + at, keyW + at, n, stage[wave], f, te);
+    ex = integrate_wave<false, PK>(P, it.t, it.X, j0, m, keys + at, keyW + at, n, (lds_u64 *)S2.stage[wave],
+                                   (lds_u64 *)S2.expTab, f, te);
   publish_spikes(P, it.t + 1, j0 + lane, f, te, it.S.popCnt, it.S.count);  // LTP follows in k_batch_ltp
   for (int o = 32; o > 0; o >>= 1) ex += __shfl_down(ex, o);
   if (lane == 0 && ex) atomicAdd(counter_slot(P.counters) + 1, ex);
@@ -2060,14 +2134,16 @@ static int build_device(dpsnn_net *n) {
   for (uint32_t s = 0; s < P.nsub; ++s) {
     const SubPop &x = n->par.sp[s];
     double *o = &sp[size_t(s) * kParams];
-    o[kTau] = x.Tau; o[kTheta] = x.Theta; o[kH] = x.H; o[kTarp] = x.Tarp;
-    o[kAlphaC] = x.AlphaC; o[kTauC] = x.TauC; o[kGC] = x.gC;
-    // div_rn needs normal divisors with normal reciprocals
+    o[kTheta] = x.Theta; o[kH] = x.H; o[kTarp] = x.Tarp;
+    o[kAlphaC] = x.AlphaC; o[kGC] = x.gC;
+    // div_short's divisors: floats (as the ini files are read), not zero
     for (double d : {x.Tau, x.TauC})
-      if (!(std::fabs(d) >= 0x1p-1021 && std::fabs(d) <= 0x1p1021))
+      if (!(std::fabs(d) > 0 && std::isfinite(d) && short_divisor(d)))
         return fail(DPSNN_ERR_CONFIG, "sub-population %u: time constant %g outside the supported range", s, d);
     o[kInvTau] = 1.0 / x.Tau;
+    o[kInvTauLo] = std::fma(-x.Tau, o[kInvTau], 1.0) / x.Tau;
     o[kInvTauC] = 1.0 / x.TauC;
+    o[kInvTauCLo] = std::fma(-x.TauC, o[kInvTauC], 1.0) / x.TauC;
   }
   double *d_sp, *d_lut, *d_inv;
   uint8_t *d_sub;
@@ -3941,9 +4017,11 @@ __global__ void k_exp(const double *x, double *y, uint64_t n) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) y[i] = dpsnn_exp(x[i]);
 }
-__global__ void k_div(const double *a, const double *b, const double *y, double *q, uint64_t n) {
+// yl[i] != 0: b[i] is a short divisor (yl = 0 goes with an exact reciprocal,
+// where both forms are one rounded product).
+__global__ void k_div(const double *a, const double *b, const double *y, const double *yl, double *q, uint64_t n) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) q[i] = div_rn(a[i], b[i], y[i]);
+  if (i < n) q[i] = yl[i] != 0.0 ? div_short(a[i], y[i], yl[i]) : div_rn(a[i], b[i], y[i]);
 }
 }  // namespace
 
@@ -4088,18 +4166,23 @@ int dpsnn_device_exp(int device, const double *x, double *y, uint64_t n) {
 int dpsnn_device_div(int device, const double *a, const double *b, double *q, uint64_t n) {
   if (!a || !b || !q) return fail(DPSNN_ERR_ARG, "null argument");
   HIP_TRY(hipSetDevice(device));
-  std::vector<double> y(n);
-  for (uint64_t i = 0; i < n; ++i) y[i] = 1.0 / b[i];  // RN(1/b), as the engine's set-up computes it
+  std::vector<double> y(n), yl(n);
+  for (uint64_t i = 0; i < n; ++i) {  // as the engine's set-up computes them
+    y[i] = 1.0 / b[i];
+    yl[i] = short_divisor(b[i]) ? std::fma(-b[i], y[i], 1.0) / b[i] : 0.0;
+  }
   double *d = nullptr;
   const size_t bytes = 8 * std::max<uint64_t>(n, 1);
-  HIP_TRY(hipMalloc((void **)&d, 4 * bytes));
+  HIP_TRY(hipMalloc((void **)&d, 5 * bytes));
   HIP_TRY(hipMemcpy(d, a, 8 * n, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(d + n, b, 8 * n, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(d + 2 * n, y.data(), 8 * n, hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(d + 3 * n, yl.data(), 8 * n, hipMemcpyHostToDevice));
   const uint64_t blocks = (n + 255) / 256;
-  if (n) hipLaunchKernelGGL(k_div, dim3((uint32_t)blocks), dim3(256), 0, 0, d, d + n, d + 2 * n, d + 3 * n, n);
+  if (n)
+    hipLaunchKernelGGL(k_div, dim3((uint32_t)blocks), dim3(256), 0, 0, d, d + n, d + 2 * n, d + 3 * n, d + 4 * n, n);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpy(q, d + 3 * n, 8 * n, hipMemcpyDeviceToHost));
+  HIP_TRY(hipMemcpy(q, d + 4 * n, 8 * n, hipMemcpyDeviceToHost));
   HIP_TRY(hipFree(d));
   return 0;
 }

@@ -68,12 +68,14 @@ DPSNN_HD static inline double dpsnn_exp_special(double tmp, uint64_t sbits, uint
   return 0x1p-1022 * y;
 }
 
-DPSNN_HD static inline double dpsnn_exp(double x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const uint64_t *T = dpsnn_exp_tab_d;
+/* Tab: the 128 (tail, bits) pairs of dpsnn_exp_table.inc, wherever the caller
+ * keeps them (the integration kernels hold a copy in LDS). */
+#if defined(__HIPCC__)
+template <class Tab>
 #else
-  const uint64_t *T = dpsnn_exp_tab_h;
+typedef const uint64_t *Tab;
 #endif
+DPSNN_HD static inline double dpsnn_exp_with(double x, Tab T) {
   const double InvLn2N = 0x1.71547652b82fep0 * 128, Shift = 0x1.8p52;
   const double NegLn2hiN = -0x1.62e42fefa0000p-8, NegLn2loN = -0x1.cf79abc9e3b3ap-47;
   const double C2 = 0x1.ffffffffffdbdp-2, C3 = 0x1.555555555543cp-3;
@@ -103,5 +105,13 @@ DPSNN_HD static inline double dpsnn_exp(double x) {
   tmp = fma(r2 * r2, fma(r, C5, C4), fma(r2, fma(r, C3, C2), tail + r));
   if (abstop == 0) return dpsnn_exp_special(tmp, sbits, ki);
   return fma(dpsnn_asf64(sbits), tmp, dpsnn_asf64(sbits));
+}
+
+DPSNN_HD static inline double dpsnn_exp(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return dpsnn_exp_with(x, dpsnn_exp_tab_d);
+#else
+  return dpsnn_exp_with(x, dpsnn_exp_tab_h);
+#endif
 }
 #endif
