@@ -300,6 +300,21 @@ struct Lifca {
   double Theta, H, Tarp, AlphaC, gC, invTau, invTauLo, invTauC, invTauCLo;
   const lds_u64 *expTab;
   uint32_t fired;
+  __device__ inline void load(const DevNet &P, uint32_t j) {
+    const double *prm = P.sp + (size_t)P.subPop[j] * kParams;
+    v = P.v[j]; c = P.c[j]; Tr = P.Tr[j]; Te = P.Te[j];
+    Theta = prm[kTheta]; H = prm[kH]; Tarp = prm[kTarp]; AlphaC = prm[kAlphaC]; gC = prm[kGC];
+    invTau = prm[kInvTau]; invTauLo = prm[kInvTauLo];
+    invTauC = prm[kInvTauC]; invTauCLo = prm[kInvTauCLo];
+  }
+  // What an event takes from the time since the one before it alone: half
+  // of it, that over Tau, and the factor c decays by.
+  __device__ inline void decay(double deltaT, double &dtHalf, double &rmHalf, double &cDecay) const {
+    dtHalf = deltaT / 2;
+    rmHalf = div_short(dtHalf, invTau, invTauLo);
+    const double rc = div_short(deltaT, invTauC, invTauCLo);
+    cDecay = 1 - rc + rc * rc / 2;
+  }
   // Both of the reference's branches (out of / in the refractory period)
   // decay c by the same expression; the out-of-refractory one also moves v.
   // The lanes of a wave take different branches, so v's update is computed
@@ -307,25 +322,27 @@ struct Lifca {
   // period: the same operations in the same order, without divergent
   // control flow.  Only the refractory exit (exp) stays a branch; it is rare.
   // A lane without an event (on = false) passes t = Tr: no time elapses, so
-  // c is multiplied by one, and v and Te are kept; nothing changes.
-  __device__ inline void event(bool on, double t, double I) {
+  // c is multiplied by one, and v and Te are kept; nothing changes.  AHEAD:
+  // dtHalf, rmHalf and cDecay are decay(t - Tr)'s, already computed.
+  template <bool AHEAD = false>
+  __device__ __attribute__((always_inline)) inline void event(bool on, double t, double I, double dtHalf = 0,
+                                                              double rmHalf = 0, double cDecay = 0) {
     double deltaT = t - Tr;
     const double TFLES = t - Te;
     const bool active = on && TFLES > Tarp;
     if (active && Tr - Te < Tarp) {
       c *= dpsnn_exp_with(div_short(-(deltaT - TFLES + Tarp), invTauC, invTauCLo), expTab);
       deltaT = TFLES - Tarp;
+      if (AHEAD) decay(deltaT, dtHalf, rmHalf, cDecay);
     }
-    const double dtHalf = deltaT / 2;
-    const double rmHalf = div_short(dtHalf, invTau, invTauLo);
-    const double rc = div_short(deltaT, invTauC, invTauCLo);
+    if (!AHEAD) decay(deltaT, dtHalf, rmHalf, cDecay);
     double w = v - v * rmHalf - gC * c * dtHalf;
     w = w - w * rmHalf - gC * c * dtHalf;
     w += I;
     // (kept here: the compiler would move v's update under a branch on
     // `active`, apart from c's, and lose what overlaps the two)
     asm volatile("" : "+v"(w));
-    c = c * (1 - rc + rc * rc / 2);
+    c = c * cDecay;
     const bool fire = active && w >= Theta;
     v = fire ? H : (active ? w : v);
     c = fire ? c + AlphaC : c;
@@ -630,6 +647,42 @@ __device__ __attribute__((always_inline)) inline bool draw_bath(Cursor &x, bool 
   return a < kNoEvent;
 }
 
+template <bool REPLAY>
+using BathCursor = std::conditional_t<REPLAY, ExtReplayCursor, ExtPhiloxCursor>;
+
+// Neuron j's bath in step t (`on`: the lane has a neuron).
+template <bool REPLAY>
+__device__ inline BathCursor<REPLAY> bath_cursor(const DevNet &P, uint32_t t, const ExtView &X, uint32_t j, bool on) {
+  BathCursor<REPLAY> x{};
+  if (on) {
+    if constexpr (REPLAY) {
+      x = ExtReplayCursor{X.time, X.value, X.off[j], X.off[j + 1]};
+    } else {
+      x.a = P.assigned[j];
+      x.inv = P.invNuExt[j];
+      x.nextF = (double)t + 1.0;
+      x.lut = P.lut + (size_t)P.subPop[j] * kLutDepth;
+      x.cap = P.maxExt[j];
+      x.nExt = 0;
+      x.onE = x.inv > 0;
+      x.R = PhiloxStream{(uint32_t)P.philoxSeed, (uint32_t)(P.philoxSeed >> 32) ^ j, P.philoxCtr[j], 0.0, 0};
+    }
+  }
+  return x;
+}
+// Leaves neuron j's bath where the step ends; returns its event count.
+template <class Cursor>
+__device__ inline uint32_t finish_bath(const DevNet &P, const ExtView &X, uint32_t j, Cursor &x) {
+  if constexpr (std::is_same_v<Cursor, ExtReplayCursor>) {
+    return x.xe - X.off[j];
+  } else {
+    x.finish();
+    P.assigned[j] = x.a;
+    P.philoxCtr[j] = x.R.ctr;
+    return x.nExt;
+  }
+}
+
 constexpr int kChunk = 8;  // internal events per lane per LDS-staged chunk
 // From step kPackT on, a scratch entry carries its weight in the low 16 bits
 // (tick << 16 | weight): for t >= 32 every tick is at most 2^47 (t + frac
@@ -758,35 +811,11 @@ __device__ __attribute__((always_inline)) inline uint32_t integrate_wave(const D
   uint64_t rk[kChunk];
   uint4 rw = make_uint4(0, 0, 0, 0);
   if (chunks) load_chunk(tileR, tileW, 0, __ballot(n > 0), rk, rw, packed);
-  Lifca L;
-  uint32_t sp = 0;
+  Lifca L{};
   L.expTab = expTab;
-  if (on) {
-    sp = P.subPop[j];
-    const double *prm = P.sp + (size_t)sp * kParams;
-    L.v = P.v[j]; L.c = P.c[j]; L.Tr = P.Tr[j]; L.Te = P.Te[j];
-    L.Theta = prm[kTheta]; L.H = prm[kH]; L.Tarp = prm[kTarp]; L.AlphaC = prm[kAlphaC]; L.gC = prm[kGC];
-    L.invTau = prm[kInvTau]; L.invTauLo = prm[kInvTauLo];
-    L.invTauC = prm[kInvTauC]; L.invTauCLo = prm[kInvTauCLo];
-  }
-  L.fired = 0;
-  std::conditional_t<REPLAY, ExtReplayCursor, ExtPhiloxCursor> bath{};
+  if (on) L.load(P, j);
+  BathCursor<REPLAY> bath = bath_cursor<REPLAY>(P, t, X, j, on);
   lds_f64 *qv = (lds_f64 *)stage + kRing * kStageRow + lane, *qt = qv + kQueue * kWave;
-  if (on) {
-    if constexpr (REPLAY) {
-      bath = ExtReplayCursor{X.time, X.value, X.off[j], X.off[j + 1]};
-    } else {
-      ExtPhiloxCursor &xp = bath;
-      xp.a = P.assigned[j];
-      xp.inv = P.invNuExt[j];
-      xp.nextF = nextF;
-      xp.lut = P.lut + (size_t)sp * kLutDepth;
-      xp.cap = P.maxExt[j];
-      xp.nExt = 0;
-      xp.onE = xp.inv > 0;
-      xp.R = PhiloxStream{(uint32_t)P.philoxSeed, (uint32_t)(P.philoxSeed >> 32) ^ j, P.philoxCtr[j], 0.0, 0};
-    }
-  }
   bool due = draw_bath(bath, on, qt, qv);  // a bath event is due after the drawn ones
   uint32_t qi = 0;                         // the next bath event
   double head = qt[0], headV = qv[0];
@@ -848,20 +877,195 @@ __device__ __attribute__((always_inline)) inline uint32_t integrate_wave(const D
   }
   uint32_t nExt = 0;
   if (on) {
-    if constexpr (REPLAY) {
-      nExt = bath.xe - X.off[j];
-    } else {
-      bath.finish();
-      nExt = bath.nExt;
-      P.assigned[j] = bath.a;
-      P.philoxCtr[j] = bath.R.ctr;
-    }
+    nExt = finish_bath(P, X, j, bath);
     P.v[j] = L.v; P.c[j] = L.c; P.Tr[j] = L.Tr; P.Te[j] = L.Te;
   }
   fired = on && L.fired != 0;
   te = L.Te;
   wave_sync();  // the stage is free again
   return nExt;
+}
+
+// Phase 2 by three waves per tile of 64 neurons (t >= kPackT): one merges
+// each neuron's internal and bath events into one sequence, the second
+// computes what each event takes from its time alone (Lifca::decay), the
+// third runs the recurrence on v and c.  They pass the events through LDS,
+// kPipe per lane and round, with one barrier a round: in round r the first
+// makes the events r, the second works on r - 1 and the third on r - 2.
+//
+// While there are fewer tiles than SIMDs a step's phase 2 is one wave's
+// instructions, about six cycles each whatever they depend on (measured: an
+// FP64 operation takes 5.4 to 6.2 cycles alone on its SIMD, in a chain or
+// not); the three waves share them almost evenly.  The work is the same plus
+// the LDS traffic, so with more tiles than the chip runs at once
+// integrate_wave is the better one (kPipeTiles).
+constexpr int kPipe = 4;
+// Tiles up to which phase 2 runs in this form: 1,250 tiles (80,000 neurons)
+// take less time in it, 2,813 tiles (180,000 neurons) more.
+constexpr uint32_t kPipeTiles = 2048;
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) f64x2 lds_f64x2;
+struct PipeLds {
+  f64x2 event[3][kPipe][kWave];   // time, value
+  f64x2 decay[2][kPipe][kWave];   // dtHalf, rmHalf
+  double cDecay[2][kPipe][kWave];
+  uint64_t expTab[kExpTab];
+  uint64_t stage[kStagePackedBytes / sizeof(uint64_t)];
+  uint32_t count[3][kWave];       // events of the lane in the round (the rest change nothing)
+  uint32_t last;                  // the last round with events
+};
+constexpr int kPipeThreads = 3 * kWave;
+
+// Barrier of a pipelined tile: LDS is ordered around it, global loads in
+// flight stay in flight.
+__device__ inline void pipe_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// As integrate_wave, for the workgroup of a tile (every wave calls it).
+// fired and te are the third wave's, the external count the first wave's.
+template <bool REPLAY>
+__device__ __attribute__((always_inline)) inline uint32_t integrate_pipe(const DevNet &P, uint32_t t, const ExtView &X, uint32_t j0,
+                                                                         uint32_t m, const uint64_t *tileK, uint32_t n,
+                                                                         PipeLds &S, bool &fired, double &te) {
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t role = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const bool on = lane < m;
+  const uint32_t j = j0 + lane;
+  lds_f64x2 *event = (lds_f64x2 *)&S.event[0][0][lane], *decay = (lds_f64x2 *)&S.decay[0][0][lane];
+  lds_f64 *cDecay = (lds_f64 *)&S.cDecay[0][0][lane];
+  typedef __attribute__((address_space(3))) uint32_t lds_u32;
+  lds_u32 *count = (lds_u32 *)&S.count[0][lane], *last = (lds_u32 *)&S.last;
+  load_exp_table((lds_u64 *)S.expTab);
+  if (threadIdx.x == 0) *last = ~0u;
+  pipe_barrier();
+  if (role == 0) {
+    if (!on) n = 0;
+    uint32_t nmax = n;
+    for (int o = 32; o > 0; o >>= 1) nmax = max(nmax, (uint32_t)__shfl_xor((int)nmax, o));
+    nmax = (uint32_t)__builtin_amdgcn_readfirstlane((int)nmax);
+    const uint64_t tBits = dpsnn_asu64((double)t);
+    const __amdgpu_buffer_rsrc_t tileR = buffer_view(wave_uniform(tileK), P.cap * kWave * (uint32_t)sizeof(uint64_t));
+    const uint32_t chunks = (nmax + kChunk - 1) / kChunk;
+    lds_u64 *ring = (lds_u64 *)S.stage;
+    lds_f64 *qv = (lds_f64 *)ring + kRing * kStageRow + lane, *qt = qv + kQueue * kWave;
+    uint64_t rk[kChunk];
+    uint4 rw = make_uint4(0, 0, 0, 0);
+    if (chunks) load_chunk(tileR, nullptr, 0, __ballot(n > 0), rk, rw, true);
+    BathCursor<REPLAY> bath = bath_cursor<REPLAY>(P, t, X, j, on);
+    double tr = on ? P.Tr[j] : 0.0;
+    bool due = draw_bath(bath, on, qt, qv);
+    uint32_t qi = 0;
+    double head = qt[0], headV = qv[0];
+    if (chunks) store_chunk(ring, nullptr, 0, rk, rw, true);
+    if (chunks > 1) {
+      load_chunk(tileR, nullptr, 1, __ballot(n > kChunk), rk, rw, true);
+      store_chunk(ring, nullptr, 1, rk, rw, true);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), as in integrate_wave
+    uint32_t staged = min(chunks, 2u), e = 0, buf = 0;
+    if (staged < chunks) load_chunk(tileR, nullptr, staged, __ballot(n > staged * kChunk), rk, rw, true);
+    wave_sync();
+    uint32_t have = min(n, staged * kChunk);
+    double without = n <= staged * kChunk ? kNoEvent : -kNoEvent;
+    uint64_t kv = ring[lane];
+    uint32_t r = 0, fin = ~0u;
+    do {
+      if (fin == ~0u) {
+        uint32_t some = 0;
+#pragma unroll
+        for (int i = 0; i < kPipe; ++i) {
+          const bool inner = e < have;
+          const double kI = dpsnn_asf64(tBits + (kv >> 16));
+          const bool outer = head < (inner ? kI : without);
+          tr = outer ? head : (inner ? kI : tr);
+          const double val = outer ? headV : (double)(((float)(int16_t)(uint16_t)kv) * P.w2f);
+          event[(buf * kPipe + i) * kWave] = f64x2{tr, val};
+          some += inner || outer ? 1u : 0u;
+          e += inner && !outer ? 1u : 0u;
+          qi += outer ? 1u : 0u;
+          kv = ring[(e % kRing) * kStageRow + lane];
+          if (due && qi == (uint32_t)kQueue) {
+            due = draw_bath(bath, true, qt, qv);
+            qi = 0;
+          }
+          head = qt[qi * kWave];
+          headV = qv[qi * kWave];
+        }
+        count[buf * kWave] = some;
+        if (staged < chunks) {
+          if (!__ballot(e < min(n, (staged - 1) * kChunk))) {
+            store_chunk(ring, nullptr, staged, rk, rw, true);
+            ++staged;
+            if (staged < chunks) load_chunk(tileR, nullptr, staged, __ballot(n > staged * kChunk), rk, rw, true);
+            wave_sync();
+            have = min(n, staged * kChunk);
+            without = n <= staged * kChunk ? kNoEvent : -kNoEvent;
+            kv = ring[(e % kRing) * kStageRow + lane];
+          }
+        } else if (!(__ballot(e < have) | __ballot(head < kNoEvent))) {
+          fin = r;
+          if (lane == 0) *last = r;
+        }
+        buf = buf == 2 ? 0 : buf + 1;
+      }
+      pipe_barrier();
+      ++r;
+    } while (fin == ~0u || r <= fin + 2);
+    const uint32_t nExt = on ? finish_bath(P, X, j, bath) : 0u;
+    fired = false;
+    return nExt;
+  }
+  Lifca L{};
+  L.expTab = (lds_u64 *)S.expTab;
+  if (on) L.load(P, j);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), as in integrate_wave
+  uint32_t r = 0, fin = ~0u, buf = 0;
+  if (role == 1) {
+    double tr = L.Tr;
+    do {
+      if (r >= 1 && (fin == ~0u || r - 1 <= fin)) {
+        const uint32_t to = (r & 1) * kPipe;
+#pragma unroll
+        for (int i = 0; i < kPipe; ++i) {
+          const double at = event[(buf * kPipe + i) * kWave].x;
+          double dtHalf, rmHalf, cd;
+          L.decay(at - tr, dtHalf, rmHalf, cd);
+          decay[(to + i) * kWave] = f64x2{dtHalf, rmHalf};
+          cDecay[(to + i) * kWave] = cd;
+          tr = at;
+        }
+        buf = buf == 2 ? 0 : buf + 1;
+      }
+      pipe_barrier();
+      ++r;
+      fin = (uint32_t)__builtin_amdgcn_readfirstlane((int)*last);
+    } while (fin == ~0u || r <= fin + 2);
+    fired = false;
+    return 0;
+  }
+  do {
+    if (r >= 2) {
+      const uint32_t from = ((r - 1) & 1) * kPipe, some = count[buf * kWave];
+#pragma unroll
+      for (int i = 0; i < kPipe; ++i) {
+        const f64x2 ev = event[(buf * kPipe + i) * kWave], d = decay[(from + i) * kWave];
+        L.event<true>((uint32_t)i < some, ev.x, ev.y, d.x, d.y, cDecay[(from + i) * kWave]);
+      }
+      buf = buf == 2 ? 0 : buf + 1;
+    }
+    pipe_barrier();
+    ++r;
+    fin = (uint32_t)__builtin_amdgcn_readfirstlane((int)*last);
+  } while (fin == ~0u || r <= fin + 2);
+  if (on) {
+    P.v[j] = L.v; P.c[j] = L.c; P.Tr[j] = L.Tr; P.Te[j] = L.Te;
+  }
+  fired = on && L.fired != 0;
+  te = L.Te;
+  return 0;
 }
 
 constexpr uint64_t kNoKey = ~0ull;
@@ -1763,6 +1967,32 @@ __global__ __launch_bounds__(kBlock) void k_integrate(DevNet P, uint32_t t, ExtV
   if (lane == 0 && ex) atomicAdd(counter_slot(P.counters) + 1, ex);
 }
 
+// k_integrate by integrate_pipe: one workgroup of three waves per tile of 64
+// neurons.
+__global__ __launch_bounds__(kPipeThreads) void k_integrate_pipe(DevNet P, uint32_t t, ExtView X, NextScan S) {
+  __shared__ PipeLds L;
+  if (P.tDev) t = *P.tDev;
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (blockIdx.x == 0 && threadIdx.x < kXcds) P.workCtr[threadIdx.x * kCtrStride] = 0;  // for the next k_gather
+  if (blockIdx.x == 0 && threadIdx.x == 0 && P.bigCount) *P.bigCount = 0;                 // for the next k_sort
+  const uint32_t j0 = blockIdx.x * kWave;
+  const uint32_t m = min((uint32_t)kWave, P.N - j0);
+  const uint32_t n = lane < m ? P.keyCount[j0 + lane] : 0u;
+  const uint64_t *tileK = P.keys + (size_t)blockIdx.x * P.cap * kWave;
+  bool f = false;
+  double te = 0.0;
+  unsigned long long ex;
+  if (P.drive == DPSNN_DRIVE_REPLAY)
+    ex = integrate_pipe<true>(P, t, X, j0, m, tileK, n, L, f, te);
+  else
+    ex = integrate_pipe<false>(P, t, X, j0, m, tileK, n, L, f, te);
+  if (wave == 2) publish_spikes(P, t + 1, j0 + lane, f, te, S.popCnt, S.count);  // LTP follows in k_ltp
+  if (wave == 0) {
+    for (int o = 32; o > 0; o >>= 1) ex += __shfl_down(ex, o);
+    if (lane == 0 && ex) atomicAdd(counter_slot(P.counters) + 1, ex);
+  }
+}
+
 // The item of global tile g: the last one with tileBegin <= g.
 __device__ inline uint32_t batch_item_of(const BatchItem *items, uint32_t count, uint32_t g) {
   uint32_t lo = 0, hi = count;
@@ -1983,6 +2213,7 @@ struct dpsnn_net {
   struct dpsnn_batch *batch = nullptr;  // stepped by this batch (its stream)
   hipStream_t ownStream = nullptr;
   bool split = false;        // k_gather + k_integrate instead of the fused k_step
+  bool pipe = false;         // k_integrate_pipe instead of k_integrate (t >= kPackT)
   uint32_t gatherGrid = 0;
   std::vector<uint16_t> inSynLocal;
   // stencil-window phase 1 (k_collect + k_sort)
@@ -2255,6 +2486,10 @@ static int build_device(dpsnn_net *n) {
   n->stdpBlocks = std::min<uint32_t>((N + 3) / 4, (uint32_t)cus * 16);
   n->split = true;
   if (const char *e = std::getenv("DPSNN_SPLIT")) n->split = std::atoi(e) != 0;
+  // DPSNN_PIPE=0/1: phase 2 in one wave or three waves per tile (tests; the
+  // results are the same)
+  n->pipe = P.NW <= kPipeTiles;
+  if (const char *e = std::getenv("DPSNN_PIPE")) n->pipe = std::atoi(e) != 0;
   if (const char *e = std::getenv("DPSNN_GRAPH")) n->graphs = std::atoi(e) != 0;
   n->gatherGrid = round_up(
       std::min<uint32_t>(N, (uint32_t)cus * resident_waves((const void *)kShapes[n->shape].gather,
@@ -2477,6 +2712,18 @@ static bool plastic_at(const dpsnn_net *n, uint32_t t) {
   return n->stdp && t >= q.startPlasticity_ms && t <= q.stopPlasticity_ms;
 }
 
+// Phase 2 of a step with packed records (t >= kPackT): by three waves per
+// tile while the tiles are few.
+static void launch_integrate(const dpsnn_net *n, const DevNet &P, uint32_t t, const ExtView &X, const NextScan &S,
+                             hipStream_t stream) {
+  if (n->pipe) {
+    hipLaunchKernelGGL(k_integrate_pipe, dim3(P.NW), dim3(kPipeThreads), 0, stream, P, t, X, S);
+  } else {
+    const uint32_t blocks = (P.N + kBlock - 1) / kBlock;
+    hipLaunchKernelGGL(k_integrate<1>, dim3(blocks), dim3(kBlock), 0, stream, P, t, X, S);
+  }
+}
+
 // Key scratch of stand-alone steps, blocked by 8 events per neuron:
 // [grid][cap/8][64][8] (fused) or [N/64][cap/8][64][8] (split).
 static int ensure_scratch(dpsnn_net *n) {
@@ -2638,8 +2885,7 @@ static void launch_window_step(const dpsnn_net *n, const DevNet &P, const StepPl
   if (!P.fuseSort)
     hipLaunchKernelGGL(K.sort, dim3(n->sortGrid), dim3(kWave), phase1_lds(kSortCap, K.B), stream, P, sp.t);
   hipLaunchKernelGGL(K.sortBig, dim3(n->sortBigGrid), dim3(kWave), phase1_lds(P.cap, K.B), stream, P, sp.t);
-  const uint32_t blocks = (P.N + kBlock - 1) / kBlock;
-  hipLaunchKernelGGL(k_integrate<1>, dim3(blocks), dim3(kBlock), 0, stream, P, sp.t, sp.X, sp.S);
+  launch_integrate(n, P, sp.t, sp.X, sp.S, stream);
   if (sp.S.ltp) hipLaunchKernelGGL(k_ltp, dim3(n->stdpBlocks), dim3(kWaveLTP), 0, stream, P, sp.t + 1);
 }
 
@@ -2654,7 +2900,7 @@ static int one_step(dpsnn_net *n, const DevNet &P) {
     hipLaunchKernelGGL(K.gather, dim3(n->gatherGrid), dim3(kWave), n->ldsBytes, n->stream, P, sp.t, sp.ltd);
     const uint32_t blocks = (P.N + kBlock - 1) / kBlock;
     if (sp.t >= kPackT)
-      hipLaunchKernelGGL(k_integrate<1>, dim3(blocks), dim3(kBlock), 0, n->stream, P, sp.t, sp.X, sp.S);
+      launch_integrate(n, P, sp.t, sp.X, sp.S, n->stream);
     else
       hipLaunchKernelGGL(k_integrate<2>, dim3(blocks), dim3(kBlock), 0, n->stream, P, sp.t, sp.X, sp.S);
     if (sp.S.ltp) hipLaunchKernelGGL(k_ltp, dim3(n->stdpBlocks), dim3(kWaveLTP), 0, n->stream, P, sp.t + 1);
@@ -2696,9 +2942,7 @@ static void launch_graph_step(dpsnn_net *n, const DevNet &G) {
   } else {
     hipLaunchKernelGGL(K.gather, dim3(n->gatherGrid), dim3(kWave), n->ldsBytes, n->stream, G, 0u, 0);
   }
-  const uint32_t blocks = (G.N + kBlock - 1) / kBlock;
-  hipLaunchKernelGGL(k_integrate<1>, dim3(blocks), dim3(kBlock), 0, n->stream, G, 0u, ExtView{nullptr, nullptr, nullptr},
-                     NextScan{nullptr, 0, 1});
+  launch_integrate(n, G, 0u, ExtView{nullptr, nullptr, nullptr}, NextScan{nullptr, 0, 1}, n->stream);
   hipLaunchKernelGGL(k_tick, dim3(1), dim3(1), 0, n->stream, n->d_t);
 }
 

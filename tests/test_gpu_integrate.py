@@ -25,8 +25,11 @@ NETWORKS = [((1, 1, 1), 1, 3.0), ((21, 21, 21), 1, 30.0), ((22, 21, 21), 1, 0.05
             ((97, 96, 47), 2, 3.0), ((150, 150, 75), 2, 12.0)]
 
 
+@pytest.mark.parametrize("pipe", ["0", "1"])
 @pytest.mark.parametrize("counts,side,nu_ext", NETWORKS)
-def test_phase2_bit_exact_vs_oracle(pkg, oracle, tmp_path, counts, side, nu_ext):
+def test_phase2_bit_exact_vs_oracle(pkg, oracle, tmp_path, monkeypatch, counts, side, nu_ext, pipe):
+    """pipe: one wave or three waves per tile from step 32 on."""
+    monkeypatch.setenv("DPSNN_PIPE", pipe)
     e, e2, i = counts
     (tmp_path / "column.txt").write_text(
         f"0 {e} 0.5 0.0 {nu_ext} 20 20 15 2 1 500 0.05\n"
@@ -35,7 +38,7 @@ def test_phase2_bit_exact_vs_oracle(pkg, oracle, tmp_path, counts, side, nu_ext)
     for f in ("connectivity.txt", "bathEfficacy.txt"):
         (tmp_path / f).write_text(open(os.path.join(pkg.config_dir("c0"), f)).read())
     pkg.apply_env(pkg.config_dir("c0"), env_CFX=side, env_CFY=side, env_totalSimTime_ms=70)
-    print(f"phase 2: {side}x{side} columns of {counts}, bath {nu_ext} Hz, 70 ms vs oracle", flush=True)
+    print(f"phase 2, pipe {pipe}: {side}x{side} columns of {counts}, bath {nu_ext} Hz, 70 ms vs oracle", flush=True)
     ora = OracleNet(oracle, str(tmp_path))
     try:
         with pkg.Network(str(tmp_path), keep_spikes=True) as net:
