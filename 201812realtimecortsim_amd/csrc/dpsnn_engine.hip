@@ -176,6 +176,8 @@ struct DevNet {
   // target-major order: synapse k of neuron j's incoming list lives at
   // incOff[j] + k; in-list items name it by k (inSyn).
   int32_t *lastSpike;      // [N] last emission step (ms) of each neuron
+  uint32_t *spikeMask;     // [N] bit b: the neuron fired in slot t1 - b (t1: the last scan)
+  int32_t *lastSpike0;     // [N] lastSpike where the block of deferred steps began (k_stdp)
   const uint64_t *incOff;  // [N+1]
   int16_t *wT;
   float *tdT, *tdPre;      // timeDerivative; tdPre: before the decay (probes)
@@ -371,7 +373,10 @@ __device__ __attribute__((always_inline)) inline uint64_t publish_spikes(const D
     if (mask && count) atomicAdd(counter_slot(P.counters) + 2, (unsigned long long)__popcll(mask));
   }
   if (j < P.N) P.teHist[(size_t)slot * P.N + j] = f ? te : kNotFired;
-  if (f && P.lastSpike) P.lastSpike[j] = (int32_t)t1;
+  if (P.spikeMask && j < P.N) {
+    P.spikeMask[j] = P.spikeMask[j] << 1 | (f ? 1u : 0u);
+    if (f) P.lastSpike[j] = (int32_t)t1;
+  }
   if (popCnt && mask) {
     // one counter update per distinct (column, sub-population) among the
     // wave's fired lanes (64 consecutive neurons span at most a few)
@@ -445,6 +450,116 @@ __global__ __launch_bounds__(kWaveLTP) void k_ltp(DevNet P, uint32_t t) {
     if ((bits[j >> 6] >> (j & 63)) & 1ull) ltp_neuron(P, t, j);
 }
 
+// The LTD and LTP of a block of K steps t0 .. t0 + K - 1 at once, after the
+// last one's phase 2 (slot t0 + K is the last scan; the steps ran without
+// LTD and LTP).  A synapse's updates depend on spike times only: it is
+// delivered in step t when its source fired in slot t - delay, and its target
+// fired in slot t + 1 or did not; spikeMask holds both for the last 32 slots.
+// Each synapse's additions are made in the order the single steps make them
+// (LTD of t, then LTP of the scan t + 1), in float, so td and last come out
+// the same bit for bit.  Plasticity is on in all K steps and at slot t0 + K,
+// and no commit falls in the block; a synapse has one in-list item (no
+// spill-over runs), so its item names all its deliveries.
+//
+// One wave per target.  It moves each synapse's td and last once a block
+// instead of once a step (LTD) and once a spike (LTP): 22 B per synapse and
+// block against about 9 B per synapse and step.  202 M synapses (180,000
+// neurons, blocks of 10 and 16 steps): 1.56 ms per block; updating step by
+// step, LTD made phase 1 take 1.78 ms a step (0.91 without it, in the window
+// form) and LTP 0.26.
+constexpr uint32_t kMaskSlots = 32;
+constexpr uint32_t kStdpBlock = 16;    // steps per block
+// Shorter runs update step by step: a block moves every synapse's td and last
+// once, about what LTD and LTP of two steps move.
+constexpr uint32_t kStdpBlockMin = 3;
+constexpr int kStdpU = 4;              // independent synapses per lane
+__global__ __launch_bounds__(kWaveLTP) void k_stdp(DevNet P, uint32_t t0, uint32_t K) {
+  __shared__ float causal[kStdpSpan], anti[kStdpSpan];
+  for (uint32_t i = threadIdx.x; i < kStdpSpan; i += blockDim.x) {
+    causal[i] = P.causal[i];
+    anti[i] = P.anti[i];
+  }
+  __syncthreads();
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
+  const uint32_t waves = (gridDim.x * blockDim.x) >> 6;
+  for (uint32_t j = wave; j < P.N; j += waves) {
+    const uint32_t mj = P.spikeMask[j];
+    // lane k: the LTD increment of step t0 + k, from the last spike at or
+    // before slot t0 + k (bits K - 1 .. K - k of mj are the slots t0 + 1 ..)
+    float av = 0.0f;
+    if (lane < K) {
+      const uint32_t y = (mj >> (K - lane)) & ((1u << lane) - 1u);
+      const int lastS = y ? (int)(t0 + lane) - __builtin_ctz(y) : P.lastSpike0[j];
+      const int dt = (int)(t0 + lane) - lastS;
+      av = dt < (int)kStdpSpan ? anti[dt] : 0.0f;
+    }
+    const uint64_t beg = P.inOff[j], sbase = P.incOff[j];
+    const uint32_t len = (uint32_t)(P.inOff[j + 1] - beg);
+    for (uint32_t base = 0; base < len; base += kStdpU * kWave) {
+      uint32_t pd[kStdpU], sy[kStdpU], z[kStdpU];
+      int32_t last[kStdpU];
+      float td[kStdpU];
+#pragma unroll
+      for (int u = 0; u < kStdpU; ++u) {
+        const uint32_t i = min(base + (uint32_t)u * kWave + lane, len - 1);
+        pd[u] = P.inPD[beg + i];
+        sy[u] = P.inSyn[beg + i];
+      }
+#pragma unroll
+      for (int u = 0; u < kStdpU; ++u) {
+        // the delivery of step t0 + k in bit 31 - k
+        z[u] = (P.spikeMask[pd[u] & 0xFFFFFFu] >> (pd[u] >> 24)) << (kMaskSlots - 1 - K);
+        last[u] = P.lastT[sbase + sy[u]];
+        td[u] = P.tdT[sbase + sy[u]];
+      }
+      for (uint32_t k = 0; k < K; ++k) {
+        const int t = (int)(t0 + k);
+        const float a = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(av), (int)k));
+#pragma unroll
+        for (int u = 0; u < kStdpU; ++u) {
+          const bool delivered = (int32_t)z[u] < 0;
+          z[u] <<= 1;
+          td[u] = delivered ? td[u] + a : td[u];
+          last[u] = delivered ? t : last[u];
+        }
+        if ((mj >> (K - 1 - k)) & 1u) {  // uniform: the target fired in slot t + 1
+#pragma unroll
+          for (int u = 0; u < kStdpU; ++u) {
+            const int dt = t - last[u];
+            const float f = causal[min((uint32_t)dt, kStdpSpan - 1)];
+            td[u] += last[u] != 0 && dt < (int)kStdpSpan ? f : 0.0f;
+          }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kStdpU; ++u)
+        if (base + (uint32_t)u * kWave + lane < len) {
+          P.lastT[sbase + sy[u]] = last[u];
+          P.tdT[sbase + sy[u]] = td[u];
+        }
+    }
+  }
+}
+
+// lastSpike0 = lastSpike.
+__global__ __launch_bounds__(kWaveLTP) void k_stdp_begin(DevNet P) {
+  const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j < P.N) P.lastSpike0[j] = P.lastSpike[j];
+}
+
+// spikeMask from the spike bitmaps (a restored network): slots t, t - 1, ...
+__global__ __launch_bounds__(kWaveLTP) void k_mask_from_bits(DevNet P, uint32_t t) {
+  const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= P.N) return;
+  uint32_t m = 0;
+  for (uint32_t b = 0; b < min(min(P.RS, kMaskSlots), t + 1); ++b) {
+    const uint64_t w = P.bits[(size_t)((t - b) & (P.RS - 1)) * P.NW + (j >> 6)];
+    m |= (uint32_t)((w >> (j & 63)) & 1ull) << b;
+  }
+  P.spikeMask[j] = m;
+}
+
 // longTermPlasticity (DPSNN_localNet_sim.c:312-414), once per simulated
 // second at ms % 1000 == 999: exc->exc synapses take w + td (+drift),
 // clipped to [0, 2J] in float and re-quantized to int16; td then decays
@@ -496,6 +611,42 @@ __global__ __launch_bounds__(kWaveLTP) void k_refresh_weights(DevNet P) {
     const uint64_t base = P.incOff[j];
     for (uint64_t it = P.inOff[j] + lane; it < P.inOff[j + 1]; it += 64)
       const_cast<int16_t *>(P.inW)[it] = P.wT[base + P.inSyn[it]];
+  }
+}
+
+// ... and so do the window layout's: one wave per (unit, pass, wave) stream,
+// a lane per chunk.  A chunk's items are its target's items of the pass's run
+// delay from 8 times its place in the target's run of chunks on; the in-list
+// is run delay descending, so the pass's first item is found by bisection.
+__global__ __launch_bounds__(kWaveLTP) void k_refresh_window(DevNet P) {
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t waves = (gridDim.x * blockDim.x) >> 6;
+  const uint32_t streams = P.winUnits * P.winPasses * kWindowWaves;
+  for (uint32_t st = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; st < streams; st += waves) {
+    const uint32_t u = st / (P.winPasses * kWindowWaves), pass = st / kWindowWaves % P.winPasses;
+    const uint32_t d = P.winPasses - 1 - pass;
+    const uint32_t col = u / P.winUnitsPerCol, j0 = col * P.npc + (u - col * P.winUnitsPerCol) * P.winUnit;
+    const uint64_t cb = P.winChunk[st], ce = P.winChunk[st + 1];
+    uint32_t carry = 0;  // chunks of the run that the next 64 chunks go on with
+    for (uint64_t c0 = cb; c0 < ce; c0 += 64) {
+      const uint64_t c = c0 + lane;
+      const uint32_t q = c < ce ? P.winDesc[c] : kWindowFirst;
+      const uint64_t first = __ballot(q >= kWindowFirst) & (~0ull >> (63 - lane));
+      const uint32_t place = first ? lane - (63 - (uint32_t)__clzll((long long)first)) : carry + lane;
+      carry = (uint32_t)__shfl((int)place, 63) + 1;
+      if (c >= ce) continue;
+      const uint32_t j = j0 + (q & kWindowTarget);
+      const uint64_t end = P.inOff[j + 1];
+      uint64_t lo = P.inOff[j], hi = end;  // first item of run delay <= d
+      while (lo < hi) {
+        const uint64_t mid = (lo + hi) / 2;
+        if ((P.inPD[mid] >> 24) > d) lo = mid + 1; else hi = mid;
+      }
+      uint32_t *item = const_cast<uint32_t *>(P.winItem) + c * kWindowChunk;
+      const uint64_t from = lo + (uint64_t)place * kWindowChunk;
+      for (uint32_t i = 0; i < kWindowChunk && from + i < end && (P.inPD[from + i] >> 24) == d; ++i)
+        item[i] = (item[i] & 0xFFFF0000u) | (uint16_t)P.inW[from + i];
+    }
   }
 }
 
@@ -2206,6 +2357,8 @@ struct dpsnn_net {
   uint32_t grid = 0;
   size_t ldsBytes = 0;
   bool stdp = false;         // plasticity runs at some step of [0, total)
+  uint32_t stdpBlock = 0;    // most steps whose LTD and LTP one k_stdp may make (0: step by step)
+  bool deferring = false;    // inside such a block
   bool uploaded = false;     // build_device done (dpsnn_upload)
   std::string outDir;        // owned copy of opt.output_dir
   uint32_t stdpBlocks = 0;
@@ -2447,6 +2600,8 @@ static int build_device(dpsnn_net *n) {
     }
     std::vector<int32_t> lastSpike(N, -100000);  // DPSNN_localNet_init.c:217
     if ((rc = dev_alloc(n, &P.lastSpike, N)) || (rc = upload(n, P.lastSpike, lastSpike.data(), N))) return rc;
+    if ((rc = dev_alloc(n, &P.lastSpike0, N)) || (rc = dev_alloc(n, &P.spikeMask, N))) return rc;
+    HIP_TRY(hipMemsetAsync(P.spikeMask, 0, 4 * (size_t)N, n->stream));
     // tables, initLongTermPlasticity DPSNN_neuron_sim.c:45-92
     std::vector<float> causal, anti;
     stdp_tables(q, causal, anti);
@@ -2486,6 +2641,14 @@ static int build_device(dpsnn_net *n) {
   n->stdpBlocks = std::min<uint32_t>((N + 3) / 4, (uint32_t)cus * 16);
   n->split = true;
   if (const char *e = std::getenv("DPSNN_SPLIT")) n->split = std::atoi(e) != 0;
+  // k_stdp's blocks: the mask holds slots t0 - delay .. t0 + K, and every
+  // synapse has one item.  DPSNN_STDP_BLOCK lowers their steps (0: step by
+  // step), for tests and timing; the results are the same
+  if (n->stdp && n->split && c.in_off[N] == c.S && c.max_delay + 1 + kStdpBlockMin < kMaskSlots) {
+    n->stdpBlock = std::min<uint32_t>(kStdpBlock, kMaskSlots - 1 - c.max_delay);
+    if (const char *e = std::getenv("DPSNN_STDP_BLOCK"))
+      n->stdpBlock = std::min<uint32_t>(n->stdpBlock, (uint32_t)std::max(0, std::atoi(e)));
+  }
   // DPSNN_PIPE=0/1: phase 2 in one wave or three waves per tile (tests; the
   // results are the same)
   n->pipe = P.NW <= kPipeTiles;
@@ -2656,6 +2819,12 @@ static int write_probe(dpsnn_net *n, const char *prefix, uint32_t sec, const flo
   return 0;
 }
 
+// The in-list items' weights (both layouts) from the synapses'.
+static void refresh_weights(dpsnn_net *n) {
+  hipLaunchKernelGGL(k_refresh_weights, dim3(n->stdpBlocks), dim3(kWaveLTP), 0, n->stream, n->dev);
+  if (n->winOn) hipLaunchKernelGGL(k_refresh_window, dim3(n->stdpBlocks), dim3(kWaveLTP), 0, n->stream, n->dev);
+}
+
 static int commit(dpsnn_net *n, uint32_t t) {
   const dpsnn_parameters &q = n->par.pub;
   const uint32_t sec = t / 1000;
@@ -2665,7 +2834,7 @@ static int commit(dpsnn_net *n, uint32_t t) {
   int rc;
   if (probes && (rc = write_probe(n, "synPeriodicProbe_A", sec, nullptr))) return rc;
   hipLaunchKernelGGL(k_commit, dim3(n->stdpBlocks), dim3(kWaveLTP), 0, n->stream, n->dev);
-  hipLaunchKernelGGL(k_refresh_weights, dim3(n->stdpBlocks), dim3(kWaveLTP), 0, n->stream, n->dev);
+  refresh_weights(n);
   HIP_TRY(hipGetLastError());
   if (probes && (rc = write_probe(n, "synPeriodicProbe_B", sec, n->dev.tdPre))) return rc;
   return 0;
@@ -2814,9 +2983,9 @@ static int pre_step(dpsnn_net *n, StepPlan &sp) {
     uint32_t rec0;
     if ((rc = open_record(n, 0, &rec0)) || (rc = compact(n, 0, rec0))) return rc;
   }
-  sp.ltd = plastic_at(n, t);
+  sp.ltd = plastic_at(n, t) && !n->deferring;
   sp.commitNow = sp.ltd && t % 1000 == 999;
-  sp.ltpNext = next < T && plastic_at(n, next);
+  sp.ltpNext = next < T && plastic_at(n, next) && !n->deferring;
   sp.recordNext = n->collect && next < T;
   sp.S = NextScan{nullptr, sp.ltpNext && !sp.commitNow, next < T};
   if (sp.recordNext) {
@@ -2927,8 +3096,31 @@ static bool graph_run_ok(const dpsnn_net *n, uint32_t steps) {
   if (!n->graphs || !n->split || n->dev.drive != DPSNN_DRIVE_PHILOX || n->collect) return false;
   if (t < kPackT || (uint64_t)t + steps >= T) return false;
   for (uint32_t k = 0; k <= steps; ++k)
-    if (plastic_at(n, t + k)) return false;
+    if (plastic_at(n, t + k) && !n->deferring) return false;
   return true;
+}
+
+// Steps from n->t on, at most `left`, that may run as one block of k_stdp:
+// plastic throughout and at the scan after them, no commit among them, the
+// run not over.
+static uint32_t stdp_block(const dpsnn_net *n, uint32_t left) {
+  const uint32_t t = n->t, T = n->par.pub.totalSimTime_ms;
+  if (!n->stdpBlock || t >= T || !plastic_at(n, t)) return 0;
+  const uint64_t stop = std::min<uint64_t>(T - 1, n->par.pub.stopPlasticity_ms);  // the last scan
+  const uint64_t K = std::min<uint64_t>({left, n->stdpBlock, 999 - t % 1000, stop - std::min<uint64_t>(stop, t)});
+  return K >= kStdpBlockMin ? (uint32_t)K : 0;
+}
+
+static void stdp_begin(dpsnn_net *n) {
+  n->deferring = true;
+  hipLaunchKernelGGL(k_stdp_begin, dim3((n->dev.N + kWaveLTP - 1) / kWaveLTP), dim3(kWaveLTP), 0, n->stream, n->dev);
+}
+static int stdp_end(dpsnn_net *n, uint32_t t0) {
+  n->deferring = false;
+  if (n->t > t0)
+    hipLaunchKernelGGL(k_stdp, dim3(n->stdpBlocks), dim3(kWaveLTP), 0, n->stream, n->dev, t0, n->t - t0);
+  HIP_TRY(hipGetLastError());
+  return 0;
 }
 
 // Launches of one plain step in the graph form (t from P.tDev).
@@ -2990,18 +3182,25 @@ static int graph_steps(dpsnn_net *n, const DevNet &P) {
 // qualify and `graphs` allows them).
 static int run_steps(dpsnn_net *n, const DevNet &P, uint32_t nsteps, bool graphs) {
   int rc;
+  uint32_t blockFrom = 0, blockLeft = 0;  // the open block of k_stdp
   for (uint32_t k = 0; k < nsteps;) {
     if (n->t >= n->par.pub.totalSimTime_ms) {
       rc = drain(n);
       return rc ? rc : DPSNN_DONE;
     }
-    if (graphs && nsteps - k >= kGraphSteps && graph_run_ok(n, kGraphSteps)) {
-      if ((rc = graph_steps(n, P))) return rc;
-      k += kGraphSteps;
-      continue;
+    if (!n->deferring && (blockLeft = stdp_block(n, nsteps - k))) {
+      blockFrom = n->t;
+      stdp_begin(n);
     }
-    if ((rc = one_step(n, P))) return rc;
-    ++k;
+    const uint32_t left = n->deferring ? blockLeft : nsteps - k;
+    const uint32_t steps = graphs && left >= kGraphSteps && graph_run_ok(n, kGraphSteps) ? kGraphSteps : 1;
+    rc = steps > 1 ? graph_steps(n, P) : one_step(n, P);
+    k += steps;
+    if (n->deferring && (rc || (blockLeft -= steps) == 0)) {
+      const int rc2 = stdp_end(n, blockFrom);
+      rc = rc ? rc : rc2;
+    }
+    if (rc) return rc;
   }
   return 0;
 }
@@ -3368,7 +3567,7 @@ uint64_t dpsnn_device_bytes_needed(const dpsnn_net *n) {
   b += r(8 * (N + 1)) + r(4 * (items + kWave)) + r(2 * items);  // in-lists
   if (n->stdp) {
     const uint64_t S = c.S;
-    b += r(8 * (N + 1)) + r(2 * S) + r(S) + r(2 * items) + 2 * r(4 * S) + r(4 * N);
+    b += r(8 * (N + 1)) + r(2 * S) + r(S) + r(2 * items) + 2 * r(4 * S) + 3 * r(4 * N);
     if (!q.statSynPeriodicProbe_writeDisable) b += r(4 * S);
     b += 2 * r(4 * kStdpSpan) + 2 * r(4 * q.subPopNumber * q.subPopNumber);
   }
@@ -3707,6 +3906,14 @@ int dpsnn_restore(const char *inidir, const dpsnn_options *opt, const char *path
   HIP_TRY(hipSetDevice(n->opt.device));
   HIP_TRY(hipStreamSynchronize(n->stream));
   if ((rc = ck_device_arrays(n, [&](auto *d, size_t cnt) { return ck_dev_read(cf.f, d, cnt); }))) return rc;
+  if (n->stdp) {
+    // what the restored arrays determine: the spike masks and, after a
+    // commit, the in-list items' weights
+    hipLaunchKernelGGL(k_mask_from_bits, dim3((n->dev.N + kWaveLTP - 1) / kWaveLTP), dim3(kWaveLTP), 0, n->stream,
+                       n->dev, h.t);
+    refresh_weights(n);
+    HIP_TRY(hipGetLastError());
+  }
   Ran3::State rs{};
   if ((rc = ck_read(cf.f, &rs, 1))) return rc;
   n->rng.set_state(rs);
