@@ -469,9 +469,12 @@ __global__ __launch_bounds__(kWaveLTP) void k_ltp(DevNet P, uint32_t t) {
 // form) and LTP 0.26.
 constexpr uint32_t kMaskSlots = 32;
 constexpr uint32_t kStdpBlock = 16;    // steps per block
-// Shorter runs update step by step: a block moves every synapse's td and last
-// once, about what LTD and LTP of two steps move.
-constexpr uint32_t kStdpBlockMin = 3;
+// A single step updates its synapses itself: a block moves every synapse's td
+// and last, one step's LTD and LTP only those of the delivered ones and of the
+// targets that spike (180,000 neurons, ms per step in calls of 3: 1.75 in
+// blocks, 2.46 step by step; 31,250 neurons: 0.52 and 0.61; calls of one: 2.5
+// and 2.46 by the kernels' times).
+constexpr uint32_t kStdpBlockMin = 2;
 constexpr int kStdpU = 4;              // independent synapses per lane
 __global__ __launch_bounds__(kWaveLTP) void k_stdp(DevNet P, uint32_t t0, uint32_t K) {
   __shared__ float causal[kStdpSpan], anti[kStdpSpan];
@@ -2358,7 +2361,8 @@ struct dpsnn_net {
   size_t ldsBytes = 0;
   bool stdp = false;         // plasticity runs at some step of [0, total)
   uint32_t stdpBlock = 0;    // most steps whose LTD and LTP one k_stdp may make (0: step by step)
-  bool deferring = false;    // inside such a block
+  bool deferring = false;    // inside such a block: its first step, and the steps left of it
+  uint32_t blockFrom = 0, blockLeft = 0;
   bool uploaded = false;     // build_device done (dpsnn_upload)
   std::string outDir;        // owned copy of opt.output_dir
   uint32_t stdpBlocks = 0;
@@ -3111,14 +3115,21 @@ static uint32_t stdp_block(const dpsnn_net *n, uint32_t left) {
   return K >= kStdpBlockMin ? (uint32_t)K : 0;
 }
 
-static void stdp_begin(dpsnn_net *n) {
+// Opens a block where the next steps (at most `left`) may run as one.
+static void stdp_open(dpsnn_net *n, uint32_t left) {
+  if (n->deferring || !(n->blockLeft = stdp_block(n, left))) return;
   n->deferring = true;
+  n->blockFrom = n->t;
   hipLaunchKernelGGL(k_stdp_begin, dim3((n->dev.N + kWaveLTP - 1) / kWaveLTP), dim3(kWaveLTP), 0, n->stream, n->dev);
 }
-static int stdp_end(dpsnn_net *n, uint32_t t0) {
+// After `steps` steps (or a failed one): the open block's updates once it is
+// complete, or cut short by the failure.
+static int stdp_close(dpsnn_net *n, uint32_t steps, bool failed) {
+  if (!n->deferring || ((n->blockLeft -= steps) != 0 && !failed)) return 0;
   n->deferring = false;
-  if (n->t > t0)
-    hipLaunchKernelGGL(k_stdp, dim3(n->stdpBlocks), dim3(kWaveLTP), 0, n->stream, n->dev, t0, n->t - t0);
+  if (n->t > n->blockFrom)
+    hipLaunchKernelGGL(k_stdp, dim3(n->stdpBlocks), dim3(kWaveLTP), 0, n->stream, n->dev, n->blockFrom,
+                       n->t - n->blockFrom);
   HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -3182,25 +3193,18 @@ static int graph_steps(dpsnn_net *n, const DevNet &P) {
 // qualify and `graphs` allows them).
 static int run_steps(dpsnn_net *n, const DevNet &P, uint32_t nsteps, bool graphs) {
   int rc;
-  uint32_t blockFrom = 0, blockLeft = 0;  // the open block of k_stdp
   for (uint32_t k = 0; k < nsteps;) {
     if (n->t >= n->par.pub.totalSimTime_ms) {
       rc = drain(n);
       return rc ? rc : DPSNN_DONE;
     }
-    if (!n->deferring && (blockLeft = stdp_block(n, nsteps - k))) {
-      blockFrom = n->t;
-      stdp_begin(n);
-    }
-    const uint32_t left = n->deferring ? blockLeft : nsteps - k;
+    stdp_open(n, nsteps - k);
+    const uint32_t left = n->deferring ? n->blockLeft : nsteps - k;
     const uint32_t steps = graphs && left >= kGraphSteps && graph_run_ok(n, kGraphSteps) ? kGraphSteps : 1;
     rc = steps > 1 ? graph_steps(n, P) : one_step(n, P);
     k += steps;
-    if (n->deferring && (rc || (blockLeft -= steps) == 0)) {
-      const int rc2 = stdp_end(n, blockFrom);
-      rc = rc ? rc : rc2;
-    }
-    if (rc) return rc;
+    const int rc2 = stdp_close(n, rc ? 0 : steps, rc != 0);
+    if (rc || rc2) return rc ? rc : rc2;
   }
   return 0;
 }
@@ -3963,7 +3967,6 @@ struct dpsnn_batch {
   size_t scratchSlots = 0;
   uint32_t scratchCap = 0;
   uint32_t totalTiles = 0;   // of all members
-  bool anyPlastic = false;   // some member has STDP (the split form then runs k_batch_ltp)
   uint32_t chunkTiles = 0;   // split form: tiles per chunk (scratch bound)
   int shape = -1;
   uint32_t wavesPerCu = 0;
@@ -3973,7 +3976,7 @@ struct dpsnn_batch {
     hipGraphExec_t exec = nullptr;
     uint32_t count = 0, tiles = 0, chunkTiles = 0, wpc = 0;
     int shape = -1;
-    bool split = false, packed = false;
+    bool split = false, packed = false, ltp = false;
   } graphs[kRing];
   bool profile = false;
   std::vector<std::pair<hipEvent_t, hipEvent_t>> ev;
@@ -4040,11 +4043,7 @@ int batch_prepare(dpsnn_batch *b) {
   }
   const uint32_t cap = batch_cap(b);
   b->totalTiles = 0;
-  b->anyPlastic = false;
-  for (auto *n : b->nets) {
-    b->totalTiles += n->dev.NW;
-    b->anyPlastic = b->anyPlastic || n->stdp;
-  }
+  for (auto *n : b->nets) b->totalTiles += n->dev.NW;
   const size_t perTile = (size_t)cap * kWave * (sizeof(uint64_t) + 2 * sizeof(int16_t));
   b->chunkTiles = (uint32_t)std::max<size_t>(1, std::min<size_t>(b->totalTiles, kBatchScratchBytes / perTile));
   const size_t fusedSlots = (size_t)round_up((uint32_t)b->cus * lds_waves(lds_bytes(cap, 64)), kXcds) * kWave;
@@ -4085,8 +4084,8 @@ uint32_t batch_waves(const dpsnn_batch *b, size_t lds) {
 // The device work of one batched step: the items of ring slot r, then either
 // the persistent fused kernel or, chunk by chunk, phase 1 and phase 2
 // (packed: every member is at t >= kPackT, so phase 2 runs its packed-only
-// instance).
-int batch_launch(dpsnn_batch *b, int r, uint32_t count, uint32_t tiles, bool packed) {
+// instance; ltp: some member's next scan runs LTP).
+int batch_launch(dpsnn_batch *b, int r, uint32_t count, uint32_t tiles, bool packed, bool ltp) {
   HIP_TRY(hipMemcpyAsync(b->d_items[r], b->h_items[r], sizeof(BatchItem) * count, hipMemcpyHostToDevice, b->stream));
   const KernelShape &K = kShapes[b->shape];
   const uint32_t cap = b->scratchCap;
@@ -4112,7 +4111,7 @@ int batch_launch(dpsnn_batch *b, int r, uint32_t count, uint32_t tiles, bool pac
       else
         hipLaunchKernelGGL(k_batch_integrate<2>, dim3(blocks), dim3(kBlock), 0, b->stream, b->d_nets, b->d_items[r],
                            count, g0, g1, cap, b->keys, b->keyW, b->keyCount, b->workCtr);
-      if (b->anyPlastic)
+      if (ltp)
         hipLaunchKernelGGL(k_batch_ltp, dim3(std::min<uint32_t>((g1 - g0) * (kWave * kWave / kWaveLTP), b->cus * 16u)),
                            dim3(kWaveLTP), 0, b->stream, b->d_nets, b->d_items[r], count, g0, g1);
     }
@@ -4130,16 +4129,16 @@ void batch_drop_graphs(dpsnn_batch *b) {
 
 // The same work replayed from a graph captured once per ring slot and launch
 // configuration (the per-step arguments live in the slot's items).
-int batch_graph_launch(dpsnn_batch *b, int r, uint32_t count, uint32_t tiles, bool packed) {
+int batch_graph_launch(dpsnn_batch *b, int r, uint32_t count, uint32_t tiles, bool packed, bool ltp) {
   dpsnn_batch::Graph &g = b->graphs[r];
   const uint32_t wpc = b->wavesPerCu;
   if (!g.exec || g.count != count || g.tiles != tiles || g.chunkTiles != b->chunkTiles || g.wpc != wpc ||
-      g.shape != b->shape || g.split != b->split || g.packed != packed) {
+      g.shape != b->shape || g.split != b->split || g.packed != packed || g.ltp != ltp) {
     if (g.exec) HIP_TRY(hipGraphExecDestroy(g.exec));
     g = dpsnn_batch::Graph{};
     hipGraph_t graph = nullptr;
     HIP_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    const int rc = batch_launch(b, r, count, tiles, packed);
+    const int rc = batch_launch(b, r, count, tiles, packed, ltp);
     const hipError_t e = hipStreamEndCapture(b->stream, &graph);
     if (rc) {
       if (graph) (void)hipGraphDestroy(graph);
@@ -4159,6 +4158,7 @@ int batch_graph_launch(dpsnn_batch *b, int r, uint32_t count, uint32_t tiles, bo
     g.shape = b->shape;
     g.split = b->split;
     g.packed = packed;
+    g.ltp = ltp;
   }
   HIP_TRY(hipGraphLaunch(g.exec, b->stream));
   return 0;
@@ -4180,7 +4180,7 @@ int batch_one_step(dpsnn_batch *b, bool *any) {
   b->plans.resize(b->active.size());
   b->windowed.clear();
   uint32_t tiles = 0, count = 0;
-  bool packed = true;
+  bool packed = true, ltp = false;
   for (size_t i = 0; i < b->active.size(); ++i) {
     dpsnn_net *n = b->active[i];
     StepPlan &sp = b->plans[i];
@@ -4192,6 +4192,7 @@ int batch_one_step(dpsnn_batch *b, bool *any) {
       continue;
     }
     packed = packed && sp.t >= kPackT;
+    ltp = ltp || sp.S.ltp;
     const uint32_t idx = (uint32_t)(std::find(b->nets.begin(), b->nets.end(), n) - b->nets.begin());
     b->h_items[r][count++] = BatchItem{sp.t, sp.ltd, sp.S, sp.X, tiles, idx};
     tiles += n->dev.NW;
@@ -4206,9 +4207,9 @@ int batch_one_step(dpsnn_batch *b, bool *any) {
     HIP_TRY(hipEventRecord(b->ev[b->evUsed].first, b->stream));
   }
   if (count && b->useGraph) {
-    if ((rc = batch_graph_launch(b, r, count, tiles, packed))) return rc;
+    if ((rc = batch_graph_launch(b, r, count, tiles, packed, ltp))) return rc;
   } else if (count) {
-    if ((rc = batch_launch(b, r, count, tiles, packed))) return rc;
+    if ((rc = batch_launch(b, r, count, tiles, packed, ltp))) return rc;
   }
   // window-form members, one after another on the batch's stream and key
   // scratch (its cap is the largest member's, so their tiles fit it)
@@ -4303,7 +4304,14 @@ int dpsnn_batch_step(dpsnn_batch *b, uint32_t nsteps) {
   HIP_TRY(hipSetDevice(b->device));
   for (uint32_t k = 0; k < nsteps; ++k) {
     bool any = false;
+    // a member's blocks are its own: each ends within this call
+    if (b->split)
+      for (auto *n : b->nets) stdp_open(n, nsteps - k);
     int rc = batch_one_step(b, &any);
+    for (auto *n : b->nets) {
+      const int rc2 = stdp_close(n, rc || !any ? 0 : 1, rc || !any);
+      rc = rc ? rc : rc2;
+    }
     if (rc) return rc;
     if (!any) {
       for (auto *n : b->nets)
