@@ -108,6 +108,12 @@ __device__ inline XcdWalk xcd_walk(uint32_t total) {
 // phase 1 was 9% slower than with the guided runs, with runs of 1 twice as
 // slow.
 constexpr uint32_t kGrabMin = 4, kGrabMax = 16;
+// Up to this many targets per wave, k_gather deals them out in a fixed strided
+// order instead: with the queue's runs of four, 5,000 targets keep half of
+// the resident waves busy with four each (ms per step, queue and fixed order:
+// 1,250 neurons 0.27 and 0.23, 5,000 neurons 0.187 and 0.163; 31,250 neurons,
+// 12 targets a wave: 0.51 and 0.55).
+constexpr uint32_t kStaticTargets = 4;
 constexpr uint32_t kCtrStride = 32;
 __device__ inline uint32_t next_item(uint32_t *ctr, uint32_t total, uint32_t &x, uint32_t home, uint32_t *last) {
   const uint32_t wavesPerXcd = max(1u, gridDim.x * (blockDim.x / 64u) / kXcds);
@@ -1714,14 +1720,18 @@ __global__ __launch_bounds__(kWave) void k_gather(DevNet P, uint32_t t, int ltd)
   unsigned long long evSum = 0;
   const uint32_t home = blockIdx.x % kXcds;
   uint32_t x = home;
-  for (uint32_t j0, j1; (j0 = next_item(P.workCtr, P.N, x, home, &j1)) < P.N;)
-    for (uint32_t j = j0; j < j1; ++j) {
+  const bool queue = P.N > kStaticTargets * gridDim.x;
+  for (uint32_t j0 = blockIdx.x, j1 = P.N;;) {
+    if (queue && (j0 = next_item(P.workCtr, P.N, x, home, &j1)) >= P.N) break;
+    for (uint32_t j = j0; j < j1; j += queue ? 1u : gridDim.x) {
       const size_t at = (size_t)(j >> 6) * P.cap * kWave + (j & 63) * kRun;  // the tile's blocked scratch
       const uint32_t n = gather_sort_neuron<K, B>(P, t, j, ltd, (uint8_t *)lds, P.cap, P.keys + at, P.keyW + at,
                                                   ltd ? P.keyPos + at : nullptr);
       if (threadIdx.x == 0) P.keyCount[j] = n;
       evSum += n;
     }
+    if (!queue) break;
+  }
   if (threadIdx.x == 0) atomicAdd(counter_slot(P.counters) + 0, evSum);
 }
 
