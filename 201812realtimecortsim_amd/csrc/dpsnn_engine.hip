@@ -208,8 +208,9 @@ struct DevNet {
   uint32_t *bigCount;        // their count (zero between steps)
   uint32_t sortCap;          // k_sort keeps targets of up to this many records (<= kSortCap)
   uint32_t fuseSort;         // 1: k_collect sorts each unit's targets itself (no k_sort)
-  // Steps replayed from a captured graph read their t here (the kernel
-  // argument is then ignored); null: t is the argument.
+  // Steps replayed from a captured graph count from the t that stands here
+  // (the kernel argument is then the step's place in the graph); null: t is
+  // the argument.
   const uint32_t *tDev;
 };
 
@@ -1716,7 +1717,7 @@ __global__ __launch_bounds__(kWave) void k_batch_step(const DevNet *nets, const 
 template <int K, int B>
 __global__ __launch_bounds__(kWave) void k_gather(DevNet P, uint32_t t, int ltd) {
   extern __shared__ uint64_t lds[];
-  if (P.tDev) t = *P.tDev;
+  if (P.tDev) t += *P.tDev;
   unsigned long long evSum = 0;
   const uint32_t home = blockIdx.x % kXcds;
   uint32_t x = home;
@@ -1819,7 +1820,7 @@ __host__ __device__ inline size_t fused_sort_stride() { return (phase1_lds(kSort
 
 __global__ __launch_bounds__(kCollectThreads) void k_collect(DevNet P, uint32_t t) {
   extern __shared__ uint64_t lds[];
-  if (P.tDev) t = *P.tDev;
+  if (P.tDev) t += *P.tDev;
   const uint32_t W = P.winSlots * P.npc;  // entry W: the padding items' (never live)
   uint64_t *win = lds;
   // per target of the unit (+ padding's slot): records so far (.x) and the
@@ -2070,7 +2071,7 @@ __device__ inline uint64_t *record_runs(const DevNet &P, uint32_t j) {
 template <int B>
 __global__ __launch_bounds__(kWave) void k_sort(DevNet P, uint32_t t) {
   extern __shared__ uint64_t lds[];
-  if (P.tDev) t = *P.tDev;
+  if (P.tDev) t += *P.tDev;
   for (uint32_t j = blockIdx.x; j < P.N; j += gridDim.x) {
     const uint32_t n = P.keyCount[j];
     if (n > P.sortCap) {
@@ -2086,7 +2087,7 @@ __global__ __launch_bounds__(kWave) void k_sort(DevNet P, uint32_t t) {
 template <int B>
 __global__ __launch_bounds__(kWave) void k_sort_big(DevNet P, uint32_t t) {
   extern __shared__ uint64_t lds[];
-  if (P.tDev) t = *P.tDev;
+  if (P.tDev) t += *P.tDev;
   if (blockIdx.x == 0 && threadIdx.x < kXcds) P.winCtr[threadIdx.x * kCtrStride] = 0;  // for the next k_collect
   const uint32_t count = *P.bigCount;
   for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
@@ -2107,7 +2108,7 @@ struct IntegrateLds {
 template <int PK>
 __global__ __launch_bounds__(kBlock) void k_integrate(DevNet P, uint32_t t, ExtView X, NextScan S) {
   __shared__ IntegrateLds<PK> S2;
-  if (P.tDev) t = *P.tDev;
+  if (P.tDev) t += *P.tDev;
   load_exp_table((lds_u64 *)S2.expTab);
   __syncthreads();
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -2135,7 +2136,7 @@ __global__ __launch_bounds__(kBlock) void k_integrate(DevNet P, uint32_t t, ExtV
 // neurons.
 __global__ __launch_bounds__(kPipeThreads) void k_integrate_pipe(DevNet P, uint32_t t, ExtView X, NextScan S) {
   __shared__ PipeLds L;
-  if (P.tDev) t = *P.tDev;
+  if (P.tDev) t += *P.tDev;
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (blockIdx.x == 0 && threadIdx.x < kXcds) P.workCtr[threadIdx.x * kCtrStride] = 0;  // for the next k_gather
   if (blockIdx.x == 0 && threadIdx.x == 0 && P.bigCount) *P.bigCount = 0;                 // for the next k_sort
@@ -2256,10 +2257,8 @@ __global__ __launch_bounds__(kWaveLTP) void k_batch_ltp(const DevNet *nets, cons
   }
 }
 
-// The step counter of graph-replayed steps: set before a replay, advanced
-// by the last node of each step.
+// The first step of a graph replay, set before it.
 __global__ void k_set_t(uint32_t *t, uint32_t v) { *t = v; }
-__global__ void k_tick(uint32_t *t) { *t += 1u; }
 
 // Fills n doubles with v.
 __global__ void k_fill_f64(double *p, double v, uint64_t n) {
@@ -3096,9 +3095,9 @@ static int one_step(dpsnn_net *n, const DevNet &P) {
 
 // ----------------------------------------------------------------------------
 // Graph-replayed steps.  kGraphSteps consecutive plain steps are captured
-// once into a HIP graph whose kernels read the step's t from the device
-// counter d_t (set before each replay, advanced by a k_tick node after each
-// step), so that the same graph replays any run of such steps.  Steps
+// once into a HIP graph whose kernels take the step's t from the device
+// word d_t (set before each replay) and their step's place in the graph, so
+// that the same graph replays any run of such steps.  Steps
 // qualify when nothing the host does around a step is needed: split form,
 // Philox drive, no raster or rates collected, no plasticity, t >= kPackT
 // (the packed scratch), and the next step still inside the run.
@@ -3144,19 +3143,18 @@ static int stdp_close(dpsnn_net *n, uint32_t steps, bool failed) {
   return 0;
 }
 
-// Launches of one plain step in the graph form (t from P.tDev).
-static void launch_graph_step(dpsnn_net *n, const DevNet &G) {
+// Launches of the graph's step k (t from G.tDev).
+static void launch_graph_step(dpsnn_net *n, const DevNet &G, uint32_t k) {
   const KernelShape &K = kShapes[n->shape];
   if (n->winOn) {
-    hipLaunchKernelGGL(k_collect, dim3(n->winGrid), dim3(kCollectThreads), n->winLds, n->stream, G, 0u);
+    hipLaunchKernelGGL(k_collect, dim3(n->winGrid), dim3(kCollectThreads), n->winLds, n->stream, G, k);
     if (!G.fuseSort)
-      hipLaunchKernelGGL(K.sort, dim3(n->sortGrid), dim3(kWave), phase1_lds(kSortCap, K.B), n->stream, G, 0u);
-    hipLaunchKernelGGL(K.sortBig, dim3(n->sortBigGrid), dim3(kWave), phase1_lds(G.cap, K.B), n->stream, G, 0u);
+      hipLaunchKernelGGL(K.sort, dim3(n->sortGrid), dim3(kWave), phase1_lds(kSortCap, K.B), n->stream, G, k);
+    hipLaunchKernelGGL(K.sortBig, dim3(n->sortBigGrid), dim3(kWave), phase1_lds(G.cap, K.B), n->stream, G, k);
   } else {
-    hipLaunchKernelGGL(K.gather, dim3(n->gatherGrid), dim3(kWave), n->ldsBytes, n->stream, G, 0u, 0);
+    hipLaunchKernelGGL(K.gather, dim3(n->gatherGrid), dim3(kWave), n->ldsBytes, n->stream, G, k, 0);
   }
-  launch_integrate(n, G, 0u, ExtView{nullptr, nullptr, nullptr}, NextScan{nullptr, 0, 1}, n->stream);
-  hipLaunchKernelGGL(k_tick, dim3(1), dim3(1), 0, n->stream, n->d_t);
+  launch_integrate(n, G, k, ExtView{nullptr, nullptr, nullptr}, NextScan{nullptr, 0, 1}, n->stream);
 }
 
 static int capture_step_graph(dpsnn_net *n, const DevNet &P) {
@@ -3172,7 +3170,7 @@ static int capture_step_graph(dpsnn_net *n, const DevNet &P) {
   G.tDev = n->d_t;
   hipGraph_t g = nullptr;
   HIP_TRY(hipStreamBeginCapture(n->stream, hipStreamCaptureModeThreadLocal));
-  for (uint32_t k = 0; k < kGraphSteps; ++k) launch_graph_step(n, G);
+  for (uint32_t k = 0; k < kGraphSteps; ++k) launch_graph_step(n, G, k);
   const hipError_t e = hipStreamEndCapture(n->stream, &g);
   if (e != hipSuccess) return fail(DPSNN_ERR_DEVICE, "graph capture of the step failed: %s", hipGetErrorString(e));
   const hipError_t ei = hipGraphInstantiate(&n->stepGraph, g, nullptr, nullptr, 0);
