@@ -164,6 +164,12 @@ struct DevNet {
   const double *lut;       // [nsub][256]
   const double *invNuExt;
   const uint32_t *maxExt;
+  // The bath of a step with packed records drawn ahead of phase 1 (k_bath),
+  // which sorts it in among the internal events; null: phase 2 draws and
+  // merges it
+  double *bathT;           // [bath cap][N] event times
+  uint32_t *bathN;         // [N] their count
+  const float *bathV;      // [nsub] their value (one per sub-population)
   double *v, *c, *Tr, *Te, *assigned;
   uint64_t *philoxCtr;
   uint64_t *bits;          // [RS][NW], RS a power of two
@@ -745,6 +751,7 @@ struct ExtReplayCursor {
   uint32_t x, xe;
   __device__ inline double at() const { return x < xe ? time[x] : kNoEvent; }
   __device__ inline double take() { return value[x++]; }
+  __device__ inline void skip() { ++x; }
   __device__ inline void finish() {}
 };
 
@@ -770,6 +777,13 @@ struct ExtPhiloxCursor {
     const double u = 1.0 - lapse;
     a += -logf((float)u) * inv;
     return val;
+  }
+  __device__ inline void skip() {  // take() without the value
+    double pick, lapse;
+    R.block(pick, lapse);
+    ++nExt;
+    const double u = 1.0 - lapse;
+    a += -logf((float)u) * inv;
   }
   __device__ inline void finish() {
     if (onE && nExt >= cap && a < nextF) {
@@ -851,6 +865,47 @@ constexpr int kChunk = 8;  // internal events per lane per LDS-staged chunk
 // steps keep the weight in its own array.
 constexpr uint32_t kPackT = 32;
 constexpr int kRun = 16;   // events per neuron run in the blocked scratch
+// Weight of a bath event's record: no synapse has it (weights are quantised
+// to at most 32767 in magnitude).
+constexpr int16_t kBathWeight = -32768;
+constexpr uint32_t kBathMax = 128;  // most bath events of a neuron and ms that k_bath takes
+// The bath of step t, one lane per neuron, into bathT and bathN; its state
+// (and its counter) are where the step ends.  REPLAY: the host's events.
+// One value per sub-population, so an event is its time.
+template <bool REPLAY>
+__device__ inline void bath_step(const DevNet &P, uint32_t t, const ExtView &X, uint32_t j) {
+  const bool on = j < P.N;
+  BathCursor<REPLAY> x = bath_cursor<REPLAY>(P, t, X, j, on);
+  uint32_t n = 0;
+  if (on) {
+    for (double a; (a = x.at()) < kNoEvent; ++n) {
+      P.bathT[(size_t)n * P.N + j] = a;
+      x.skip();
+    }
+    P.bathN[j] = n;
+  }
+  unsigned long long ex = on ? finish_bath(P, X, j, x) : 0u;
+  for (int o = 32; o > 0; o >>= 1) ex += __shfl_down(ex, o);
+  if ((threadIdx.x & 63) == 0 && ex) atomicAdd(counter_slot(P.counters) + 1, ex);
+}
+__global__ __launch_bounds__(kWave) void k_bath(DevNet P, uint32_t t, ExtView X) {
+  if (P.tDev) t += *P.tDev;
+  const uint32_t j = blockIdx.x * kWave + threadIdx.x;
+  if (P.drive == DPSNN_DRIVE_REPLAY)
+    bath_step<true>(P, t, X, j);
+  else
+    bath_step<false>(P, t, X, j);
+}
+
+// The bath events of neuron j that phase 1 of step t sorts in (uniform j).
+__device__ inline uint32_t bath_count(const DevNet &P, uint32_t t, uint32_t j) {
+  return P.bathT && t >= kPackT ? P.bathN[j] : 0u;
+}
+// The tick of its event i.
+__device__ inline uint64_t bath_tick(const DevNet &P, uint64_t tBits, uint32_t j, uint32_t i) {
+  return dpsnn_asu64(P.bathT[(size_t)i * P.N + j]) - tBits;
+}
+
 // LDS of one wave in phase 2: a ring of two chunks of 64 lanes' ticks, a row
 // of kStageRow per event, then the bath queue (values, then times and their
 // end mark: [kQueue][64] and [kQueue + 1][64] doubles) and, for steps before kPackT, the
@@ -949,8 +1004,9 @@ __device__ inline void load_exp_table(lds_u64 *tab) {
 //  * is one straight block: a lane without an event runs one that changes
 //    nothing; drawing more of the bath and the refractory exit are the only
 //    branches, and rare.
-// Measured, us per launch, before and after: 5,000 neurons 208 -> 145,
-// 80,000 neurons 308 -> 226, 720,000 neurons 1155 -> 964.
+// Measured, us per launch, against a loop with those loads and chunk by chunk:
+// 5,000 neurons 145 (208), 80,000 neurons 226 (308), 720,000 neurons 964
+// (1155).
 template <bool REPLAY, int PK = 2>
 __device__ __attribute__((always_inline)) inline uint32_t integrate_wave(const DevNet &P, uint32_t t, const ExtView &X, uint32_t j0, uint32_t m,
                                           const uint64_t *tileK, const int16_t *tileW, uint32_t n, lds_u64 *stage,
@@ -1047,35 +1103,100 @@ __device__ __attribute__((always_inline)) inline uint32_t integrate_wave(const D
   return nExt;
 }
 
-// Phase 2 by three waves per tile of 64 neurons (t >= kPackT): one merges
-// each neuron's internal and bath events into one sequence, the second
-// computes what each event takes from its time alone (Lifca::decay), the
-// third runs the recurrence on v and c.  They pass the events through LDS,
-// kPipe per lane and round, with one barrier a round: in round r the first
-// makes the events r, the second works on r - 1 and the third on r - 2.
+// The time and value of a record of phase 1 with the bath sorted in
+// (t >= kPackT).
+__device__ inline double record_time(uint64_t tBits, uint64_t kv) { return dpsnn_asf64(tBits + (kv >> 16)); }
+__device__ inline float record_value(uint64_t kv, float w2f, float bathV) {
+  const int16_t w = (int16_t)(uint16_t)kv;
+  return w == kBathWeight ? bathV : ((float)w) * w2f;
+}
+
+// Phase 2 over records that hold the bath too: integrate_wave without the
+// merge.  Every lane is at the same event, so a chunk is stored over the one
+// before when the wave is done with that.  Whole wave, uniform.  Bound by
+// instruction issue (about 57 an event against 75 with the merge).  us per
+// launch, with the merge and without: 5,000 neurons 145 and 89, 80,000
+// neurons 226 and 148, 720,000 neurons 964 and 689 (k_bath 6, 8 and 22).
+__device__ __attribute__((always_inline)) inline void integrate_records(const DevNet &P, uint32_t t, uint32_t j0, uint32_t m,
+                                                                        const uint64_t *tileK, uint32_t n, lds_u64 *stage,
+                                                                        const lds_u64 *expTab, bool &fired, double &te) {
+  const uint32_t lane = threadIdx.x & 63;
+  const bool on = lane < m;
+  const uint32_t j = j0 + lane;
+  if (!on) n = 0;
+  uint32_t nmax = n;
+  for (int o = 32; o > 0; o >>= 1) nmax = max(nmax, (uint32_t)__shfl_xor((int)nmax, o));
+  nmax = (uint32_t)__builtin_amdgcn_readfirstlane((int)nmax);
+  const uint64_t tBits = dpsnn_asu64((double)t);
+  const __amdgpu_buffer_rsrc_t tileR = buffer_view(wave_uniform(tileK), P.cap * kWave * (uint32_t)sizeof(uint64_t));
+  const uint32_t chunks = (nmax + kChunk - 1) / kChunk;
+  uint64_t rk[kChunk];
+  uint4 rw = make_uint4(0, 0, 0, 0);
+  if (chunks) load_chunk(tileR, nullptr, 0, __ballot(n > 0), rk, rw, true);
+  Lifca L{};
+  L.expTab = expTab;
+  float bathV = 0.0f;
+  if (on) {
+    L.load(P, j);
+    bathV = P.bathV[P.subPop[j]];
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), as in integrate_wave
+  if (chunks) store_chunk(stage, nullptr, 0, rk, rw, true);
+  for (uint32_t c = 0; c < chunks; ++c) {
+    if (c + 1 < chunks) load_chunk(tileR, nullptr, c + 1, __ballot(n > (c + 1) * kChunk), rk, rw, true);
+    wave_sync();
+    const uint32_t from = c * kChunk, turns = min((uint32_t)kChunk, nmax - from);
+    uint64_t kv = stage[lane];
+    for (uint32_t e = 0; e < turns; ++e) {
+      const bool some = from + e < n;
+      const double at = some ? record_time(tBits, kv) : L.Tr;
+      const double val = (double)record_value(kv, P.w2f, bathV);
+      kv = stage[min(e + 1, (uint32_t)kChunk - 1) * kStageRow + lane];
+      L.event(some, at, val);
+    }
+    wave_sync();
+    if (c + 1 < chunks) store_chunk(stage, nullptr, 0, rk, rw, true);
+  }
+  if (on) {
+    P.v[j] = L.v; P.c[j] = L.c; P.Tr[j] = L.Tr; P.Te[j] = L.Te;
+  }
+  fired = on && L.fired != 0;
+  te = L.Te;
+  wave_sync();  // the stage is free again
+}
+
+// The same by three waves per tile: two compute, each for half of the tile's
+// neurons, what an event takes from its time alone (Lifca::decay), the third
+// runs the recurrence on v and c for all of them.  In round c the first two
+// put chunk c into LDS and the third works on chunk c - 1, one barrier a
+// round.  A lane of the first two holds, in register r, event lane % 8 of
+// neuron 8 r + lane / 8, as the loads deliver them; the time before an event
+// is the lane's below (the first event's: the last of the chunk before).
 //
 // While there are fewer tiles than SIMDs a step's phase 2 is one wave's
-// instructions, about six cycles each whatever they depend on (measured: an
-// FP64 operation takes 5.4 to 6.2 cycles alone on its SIMD, in a chain or
-// not); the three waves share them almost evenly.  The work is the same plus
-// the LDS traffic, so with more tiles than the chip runs at once
-// integrate_wave is the better one (kPipeTiles).
-constexpr int kPipe = 4;
-// Tiles up to which phase 2 runs in this form: 1,250 tiles (80,000 neurons)
-// take less time in it, 2,813 tiles (180,000 neurons) more.
-constexpr uint32_t kPipeTiles = 2048;
+// instructions, whatever they depend on (measured: a lone wave issues an
+// FP64, a 64-bit integer or a compare instruction at the same rate in a chain
+// or not, and a branch that a mask decides costs it more than ten), so the
+// chain is left with the instructions that need v or c.  us per launch here
+// and in integrate_records: 1,250 and 5,000 neurons 79 and 89, 31,250 neurons
+// (489 tiles) 129 and 129, 80,000 neurons 261 and 148 (the work is more, with
+// its LDS traffic, and four workgroups fit a CU); hence kPipeTiles.
 typedef double f64x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) f64x2 lds_f64x2;
-struct PipeLds {
-  f64x2 event[3][kPipe][kWave];   // time, value
-  f64x2 decay[2][kPipe][kWave];   // dtHalf, rmHalf
-  double cDecay[2][kPipe][kWave];
+typedef __attribute__((address_space(3))) float lds_f32;
+struct RecordsLds {
   uint64_t expTab[kExpTab];
-  uint64_t stage[kStagePackedBytes / sizeof(uint64_t)];
-  uint32_t count[3][kWave];       // events of the lane in the round (the rest change nothing)
-  uint32_t last;                  // the last round with events
+  uint64_t stage[kBlock / kWave][kChunk * kStageRow];
+};
+struct PipeLds {
+  f64x2 decay[2][kChunk][kWave];  // dtHalf, rmHalf
+  double cDecay[2][kChunk][kWave];
+  double time[2][kChunk][kWave];
+  float value[2][kChunk][kWave];
+  uint64_t expTab[kExpTab];
 };
 constexpr int kPipeThreads = 3 * kWave;
+constexpr uint32_t kPipeTiles = 256;
 
 // Barrier of a pipelined tile: LDS is ordered around it, global loads in
 // flight stay in flight.
@@ -1085,148 +1206,123 @@ __device__ inline void pipe_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// As integrate_wave, for the workgroup of a tile (every wave calls it).
-// fired and te are the third wave's, the external count the first wave's.
-template <bool REPLAY>
-__device__ __attribute__((always_inline)) inline uint32_t integrate_pipe(const DevNet &P, uint32_t t, const ExtView &X, uint32_t j0,
-                                                                         uint32_t m, const uint64_t *tileK, uint32_t n,
-                                                                         PipeLds &S, bool &fired, double &te) {
+__device__ __attribute__((always_inline)) inline void integrate_pipe(const DevNet &P, uint32_t t, uint32_t j0, uint32_t m,
+                                                                     const uint64_t *tileK, uint32_t n, PipeLds &S,
+                                                                     bool &fired, double &te) {
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t role = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const bool on = lane < m;
-  const uint32_t j = j0 + lane;
-  lds_f64x2 *event = (lds_f64x2 *)&S.event[0][0][lane], *decay = (lds_f64x2 *)&S.decay[0][0][lane];
-  lds_f64 *cDecay = (lds_f64 *)&S.cDecay[0][0][lane];
-  typedef __attribute__((address_space(3))) uint32_t lds_u32;
-  lds_u32 *count = (lds_u32 *)&S.count[0][lane], *last = (lds_u32 *)&S.last;
+  if (lane >= m) n = 0;
+  uint32_t nmax = n;
+  for (int o = 32; o > 0; o >>= 1) nmax = max(nmax, (uint32_t)__shfl_xor((int)nmax, o));
+  const uint32_t chunks = (uint32_t)__builtin_amdgcn_readfirstlane((int)((nmax + kChunk - 1) / kChunk));
   load_exp_table((lds_u64 *)S.expTab);
-  if (threadIdx.x == 0) *last = ~0u;
-  pipe_barrier();
-  if (role == 0) {
-    if (!on) n = 0;
-    uint32_t nmax = n;
-    for (int o = 32; o > 0; o >>= 1) nmax = max(nmax, (uint32_t)__shfl_xor((int)nmax, o));
-    nmax = (uint32_t)__builtin_amdgcn_readfirstlane((int)nmax);
+  fired = false;
+  te = 0.0;
+  if (role < 2) {
+    constexpr int R = kChunk / 2;
     const uint64_t tBits = dpsnn_asu64((double)t);
     const __amdgpu_buffer_rsrc_t tileR = buffer_view(wave_uniform(tileK), P.cap * kWave * (uint32_t)sizeof(uint64_t));
-    const uint32_t chunks = (nmax + kChunk - 1) / kChunk;
-    lds_u64 *ring = (lds_u64 *)S.stage;
-    lds_f64 *qv = (lds_f64 *)ring + kRing * kStageRow + lane, *qt = qv + kQueue * kWave;
-    uint64_t rk[kChunk];
-    uint4 rw = make_uint4(0, 0, 0, 0);
-    if (chunks) load_chunk(tileR, nullptr, 0, __ballot(n > 0), rk, rw, true);
-    BathCursor<REPLAY> bath = bath_cursor<REPLAY>(P, t, X, j, on);
-    double tr = on ? P.Tr[j] : 0.0;
-    bool due = draw_bath(bath, on, qt, qv);
-    uint32_t qi = 0;
-    double head = qt[0], headV = qv[0];
-    if (chunks) store_chunk(ring, nullptr, 0, rk, rw, true);
-    if (chunks > 1) {
-      load_chunk(tileR, nullptr, 1, __ballot(n > kChunk), rk, rw, true);
-      store_chunk(ring, nullptr, 1, rk, rw, true);
-    }
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), as in integrate_wave
-    uint32_t staged = min(chunks, 2u), e = 0, buf = 0;
-    if (staged < chunks) load_chunk(tileR, nullptr, staged, __ballot(n > staged * kChunk), rk, rw, true);
-    wave_sync();
-    uint32_t have = min(n, staged * kChunk);
-    double without = n <= staged * kChunk ? kNoEvent : -kNoEvent;
-    uint64_t kv = ring[lane];
-    uint32_t r = 0, fin = ~0u;
-    do {
-      if (fin == ~0u) {
-        uint32_t some = 0;
+    const uint32_t e = lane & 7, q0 = role * R * 8 + (lane >> 3);  // neuron of register r: q0 + 8 r
+    // per register: the neuron's reciprocals, bath value, record count, and
+    // the time its chunk before ended at
+    Lifca L[R];
+    double tr[R];
+    float bathV[R];
+    uint32_t nq[R];
 #pragma unroll
-        for (int i = 0; i < kPipe; ++i) {
-          const bool inner = e < have;
-          const double kI = dpsnn_asf64(tBits + (kv >> 16));
-          const bool outer = head < (inner ? kI : without);
-          tr = outer ? head : (inner ? kI : tr);
-          const double val = outer ? headV : (double)(((float)(int16_t)(uint16_t)kv) * P.w2f);
-          event[(buf * kPipe + i) * kWave] = f64x2{tr, val};
-          some += inner || outer ? 1u : 0u;
-          e += inner && !outer ? 1u : 0u;
-          qi += outer ? 1u : 0u;
-          kv = ring[(e % kRing) * kStageRow + lane];
-          if (due && qi == (uint32_t)kQueue) {
-            due = draw_bath(bath, true, qt, qv);
-            qi = 0;
-          }
-          head = qt[qi * kWave];
-          headV = qv[qi * kWave];
+    for (int r = 0; r < R; ++r) {
+      const uint32_t q = q0 + 8 * r;
+      nq[r] = (uint32_t)__shfl((int)n, (int)q);
+      const uint32_t jq = j0 + min(q, m - 1), sp = P.subPop[jq];
+      const double *prm = P.sp + (size_t)sp * kParams;
+      L[r].invTau = prm[kInvTau]; L[r].invTauLo = prm[kInvTauLo];
+      L[r].invTauC = prm[kInvTauC]; L[r].invTauCLo = prm[kInvTauCLo];
+      bathV[r] = P.bathV[sp];
+      tr[r] = P.Tr[jq];
+    }
+    uint64_t rk[R];
+    const auto load = [&](uint32_t c) {  // records past a neuron's last are not fetched
+      const uint32_t blk = (c * kChunk / kRun) * (kWave * kRun) + (c * kChunk) % kRun;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const uint32_t off = (blk + (q0 + 8 * r) * kRun + e) * 8u;
+        const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(tileR, c * kChunk < nq[r] ? off : kDropOffset, 0, 0);
+        rk[r] = (uint64_t)v.x | ((uint64_t)v.y << 32);
+      }
+    };
+    if (chunks) load(0);
+    pipe_barrier();
+    for (uint32_t c = 0; c <= chunks; ++c) {
+      if (c < chunks) {
+        const uint32_t half = c & 1;
+        lds_f64x2 *decay = (lds_f64x2 *)&S.decay[half][e][q0];
+        lds_f64 *cDecay = (lds_f64 *)&S.cDecay[half][e][q0], *time = (lds_f64 *)&S.time[half][e][q0];
+        lds_f32 *value = (lds_f32 *)&S.value[half][e][q0];
+        double at[R];
+        float val[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          if (c) tr[r] = ((const lds_f64 *)&S.time[half ^ 1][kChunk - 1][q0])[8 * r];
+          at[r] = record_time(tBits, rk[r]);
+          val[r] = record_value(rk[r], P.w2f, bathV[r]);
         }
-        count[buf * kWave] = some;
-        if (staged < chunks) {
-          if (!__ballot(e < min(n, (staged - 1) * kChunk))) {
-            store_chunk(ring, nullptr, staged, rk, rw, true);
-            ++staged;
-            if (staged < chunks) load_chunk(tileR, nullptr, staged, __ballot(n > staged * kChunk), rk, rw, true);
-            wave_sync();
-            have = min(n, staged * kChunk);
-            without = n <= staged * kChunk ? kNoEvent : -kNoEvent;
-            kv = ring[(e % kRing) * kStageRow + lane];
+        if (__ballot(n < (c + 1) * kChunk)) {
+          // past its last event a neuron stays where it is: the time of that
+          // event (or of the chunk before), a value that changes nothing
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            const uint32_t left = nq[r] - min(nq[r], c * kChunk);
+            const double stay = __shfl(at[r], (int)((lane & 56) + (left && left < 8 ? left - 1 : 0)));
+            at[r] = e < left ? at[r] : (left ? stay : tr[r]);
+            val[r] = e < left ? val[r] : -0.0f;
           }
-        } else if (!(__ballot(e < have) | __ballot(head < kNoEvent))) {
-          fin = r;
-          if (lane == 0) *last = r;
         }
-        buf = buf == 2 ? 0 : buf + 1;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const uint64_t ab = dpsnn_asu64(at[r]);
+          // the lane below's time (row_shr:1)
+          const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)ab, 0x111, 0xf, 0xf, false);
+          const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(ab >> 32), 0x111, 0xf, 0xf, false);
+          const double below = dpsnn_asf64((uint64_t)hi << 32 | lo);
+          double dtHalf, rmHalf, cd;
+          L[r].decay(at[r] - (e ? below : tr[r]), dtHalf, rmHalf, cd);
+          decay[8 * r] = f64x2{dtHalf, rmHalf};
+          cDecay[8 * r] = cd;
+          time[8 * r] = at[r];
+          value[8 * r] = val[r];
+        }
+        if (c + 1 < chunks) load(c + 1);
       }
       pipe_barrier();
-      ++r;
-    } while (fin == ~0u || r <= fin + 2);
-    const uint32_t nExt = on ? finish_bath(P, X, j, bath) : 0u;
-    fired = false;
-    return nExt;
+    }
+    return;
   }
   Lifca L{};
   L.expTab = (lds_u64 *)S.expTab;
+  const bool on = lane < m;
+  const uint32_t j = j0 + lane;
   if (on) L.load(P, j);
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), as in integrate_wave
-  uint32_t r = 0, fin = ~0u, buf = 0;
-  if (role == 1) {
-    double tr = L.Tr;
-    do {
-      if (r >= 1 && (fin == ~0u || r - 1 <= fin)) {
-        const uint32_t to = (r & 1) * kPipe;
+  pipe_barrier();
+  for (uint32_t round = 0; round <= chunks; ++round) {
+    if (round) {
+      const uint32_t c = round - 1, half = c & 1, left = n - min(n, c * (uint32_t)kChunk);
+      const lds_f64x2 *decay = (const lds_f64x2 *)&S.decay[half][0][lane];
+      const lds_f64 *cDecay = (const lds_f64 *)&S.cDecay[half][0][lane], *time = (const lds_f64 *)&S.time[half][0][lane];
+      const lds_f32 *value = (const lds_f32 *)&S.value[half][0][lane];
 #pragma unroll
-        for (int i = 0; i < kPipe; ++i) {
-          const double at = event[(buf * kPipe + i) * kWave].x;
-          double dtHalf, rmHalf, cd;
-          L.decay(at - tr, dtHalf, rmHalf, cd);
-          decay[(to + i) * kWave] = f64x2{dtHalf, rmHalf};
-          cDecay[(to + i) * kWave] = cd;
-          tr = at;
-        }
-        buf = buf == 2 ? 0 : buf + 1;
+      for (uint32_t i = 0; i < (uint32_t)kChunk; ++i) {
+        const f64x2 d = decay[i * kWave];
+        L.event<true>(i < left, time[i * kWave], (double)value[i * kWave], d.x, d.y, cDecay[i * kWave]);
       }
-      pipe_barrier();
-      ++r;
-      fin = (uint32_t)__builtin_amdgcn_readfirstlane((int)*last);
-    } while (fin == ~0u || r <= fin + 2);
-    fired = false;
-    return 0;
-  }
-  do {
-    if (r >= 2) {
-      const uint32_t from = ((r - 1) & 1) * kPipe, some = count[buf * kWave];
-#pragma unroll
-      for (int i = 0; i < kPipe; ++i) {
-        const f64x2 ev = event[(buf * kPipe + i) * kWave], d = decay[(from + i) * kWave];
-        L.event<true>((uint32_t)i < some, ev.x, ev.y, d.x, d.y, cDecay[(from + i) * kWave]);
-      }
-      buf = buf == 2 ? 0 : buf + 1;
     }
     pipe_barrier();
-    ++r;
-    fin = (uint32_t)__builtin_amdgcn_readfirstlane((int)*last);
-  } while (fin == ~0u || r <= fin + 2);
+  }
   if (on) {
     P.v[j] = L.v; P.c[j] = L.c; P.Tr[j] = L.Tr; P.Te[j] = L.Te;
   }
   fired = on && L.fired != 0;
   te = L.Te;
-  return 0;
 }
 
 constexpr uint64_t kNoKey = ~0ull;
@@ -1275,6 +1371,7 @@ __device__ inline float ltd_increment(const DevNet &P, uint32_t t, uint32_t j) {
 __device__ __attribute__((always_inline)) inline void ltd_neuron(const DevNet &P, uint32_t t, uint32_t j, float a, uint32_t n, const uint16_t *pos) {
   const uint32_t lane = threadIdx.x & 63;
   const uint64_t beg = P.inOff[j], sbase = P.incOff[j];
+  const uint32_t len = (uint32_t)(P.inOff[j + 1] - beg);  // positions from len on are bath events
   constexpr int U = 4;
   for (uint32_t i0 = lane; i0 < n; i0 += U * kWave) {
     uint32_t p[U], sy[U];
@@ -1282,15 +1379,15 @@ __device__ __attribute__((always_inline)) inline void ltd_neuron(const DevNet &P
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint32_t i = i0 + (uint32_t)u * kWave;
-      p[u] = i < n ? pos[(size_t)(i / kRun) * (kWave * kRun) + (i % kRun)] : 0u;
+      p[u] = i < n ? pos[(size_t)(i / kRun) * (kWave * kRun) + (i % kRun)] : len;
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u) sy[u] = i0 + (uint32_t)u * kWave < n ? P.inSyn[beg + p[u]] : 0u;
+    for (int u = 0; u < U; ++u) sy[u] = p[u] < len ? P.inSyn[beg + p[u]] : 0u;
 #pragma unroll
-    for (int u = 0; u < U; ++u) td[u] = i0 + (uint32_t)u * kWave < n ? P.tdT[sbase + sy[u]] : 0.0f;
+    for (int u = 0; u < U; ++u) td[u] = p[u] < len ? P.tdT[sbase + sy[u]] : 0.0f;
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (i0 + (uint32_t)u * kWave < n) {
+      if (p[u] < len) {
         P.lastT[sbase + sy[u]] = (int32_t)t;
         P.tdT[sbase + sy[u]] = td[u] + a;
       }
@@ -1469,10 +1566,33 @@ __device__ __attribute__((always_inline)) inline void rank_in_buckets(const uint
   }
 }
 
+// A target's bath events among the keys to be sorted: lane's events lane and
+// lane + 64, position `from` + event (after every internal one, so that equal
+// times keep internal events first), weight kBathWeight in ldsW.
+static_assert(kBathMax <= 2 * kWave, "two bath keys per lane");
+template <int B>
+__device__ __attribute__((always_inline)) inline void bath_keys(const DevNet &P, uint64_t tBits, uint32_t j, uint32_t nb,
+                                                                uint32_t from, int shift, uint32_t *bcnt, int16_t *ldsW,
+                                                                uint64_t (&key)[2]) {
+  const uint32_t lane = threadIdx.x & 63;
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const uint32_t i = lane + (uint32_t)r * kWave;
+    key[r] = kNoKey;
+    if ((uint32_t)r * kWave < nb && i < nb) {
+      const uint64_t tick = bath_tick(P, tBits, j, i);
+      key[r] = tick << 12 | (from + i);
+      ldsW[from + i] = kBathWeight;
+      atomicAdd(&bcnt[key_bucket<B>(tick, shift)], 1u);
+    }
+  }
+}
+
 // Phase 1 for neuron j, whole wave: live keys of its in-list, bucket-sorted
 // in LDS (lds: sorted[cap], ldsW[cap], bcnt[B + 1]), stored in arrival order
 // as ticks relative to bits(t) (outK) with their weights (outW) and, with
-// plastic, their in-list positions (outP, for LTD); returns n.
+// plastic, their in-list positions (outP, for LTD); returns their count n and
+// stores the count of records, with the bath's (bath_count), in *total.
 // The scratch of a tile of 64 neurons is blocked by runs of kRun events:
 // event i of neuron q at [i / kRun][q][i % kRun] (a neuron's keys fill whole
 // 128-byte lines), and outK/outW point at neuron q's [0][q][0].
@@ -1486,7 +1606,8 @@ __device__ __attribute__((always_inline)) inline void rank_in_buckets(const uint
 // on the general path.
 template <int K, int B>
 __device__ __attribute__((always_inline)) inline uint32_t gather_sort_neuron(const DevNet &P, uint32_t t, uint32_t j, int plastic, uint8_t *lds,
-                                              uint32_t cap, uint64_t *outK, int16_t *outW, uint16_t *outP) {
+                                              uint32_t cap, uint64_t *outK, int16_t *outW, uint16_t *outP,
+                                              uint32_t *total) {
   static_assert(B % kWave == 0, "bucket count must be a multiple of 64");
   constexpr int LOG2B = B == 64 ? 6 : B == 128 ? 7 : B == 256 ? 8 : B == 512 ? 9 : 10;
   uint64_t *sorted = (uint64_t *)lds;
@@ -1559,6 +1680,9 @@ __device__ __attribute__((always_inline)) inline uint32_t gather_sort_neuron(con
     for (uint32_t base = 0; base < len; base += kSuper)
       n += gather_keys<kSlowK, B>(P, t, j, beg, len, base, k8, bcnt, ldsW, shift, tBits, true, plastic);
   }
+  const uint32_t nb = bath_count(P, t, j), all = n + nb;
+  uint64_t bk[2];
+  bath_keys<B>(P, tBits, j, nb, len, shift, bcnt, ldsW, bk);
   wave_sync();
   bucket_scan<B>(bcnt);
   wave_sync();
@@ -1576,8 +1700,9 @@ __device__ __attribute__((always_inline)) inline uint32_t gather_sort_neuron(con
       scatter_keys<kSlowK, B>(k8, bcnt, sorted, shift);
     }
   }
+  if (nb) scatter_keys<2, B>(bk, bcnt, sorted, shift);
   wave_sync();
-  rank_in_buckets<B>(sorted, bcnt, n, shift, [&](uint64_t x, uint32_t p) {
+  rank_in_buckets<B>(sorted, bcnt, all, shift, [&](uint64_t x, uint32_t p) {
     const size_t at = run_offset(p);
     const int16_t wv = ldsW[x & 0xFFFu];
     if (t >= kPackT) {
@@ -1589,7 +1714,8 @@ __device__ __attribute__((always_inline)) inline uint32_t gather_sort_neuron(con
     if (plastic && !fast) outP[at] = (uint16_t)(x & 0xFFFu);
   });
   wave_sync();
-  if (plastic && !fast) ltd_neuron(P, t, j, ltd_increment(P, t, j), n, outP);
+  if (plastic && !fast) ltd_neuron(P, t, j, ltd_increment(P, t, j), all, outP);
+  if (lane == 0) *total = all;
   return n;
 }
 
@@ -1623,10 +1749,8 @@ __device__ __attribute__((always_inline)) inline unsigned long long step_tile(co
   const uint32_t m = min((uint32_t)kWave, P.N - j0);
   unsigned long long evSum = 0;
   for (uint32_t q = 0; q < m; ++q) {
-    const uint32_t n =
-        gather_sort_neuron<K, B>(P, t, j0 + q, ltd, lds, cap, wkeys + q * kRun, wW + q * kRun, wP + q * kRun);
-    if (lane == 0) wcnt[q] = n;
-    evSum += n;
+    evSum += gather_sort_neuron<K, B>(P, t, j0 + q, ltd, lds, cap, wkeys + q * kRun, wW + q * kRun, wP + q * kRun,
+                                      wcnt + q);
   }
   __threadfence_block();
   __syncthreads();
@@ -1726,10 +1850,8 @@ __global__ __launch_bounds__(kWave) void k_gather(DevNet P, uint32_t t, int ltd)
     if (queue && (j0 = next_item(P.workCtr, P.N, x, home, &j1)) >= P.N) break;
     for (uint32_t j = j0; j < j1; j += queue ? 1u : gridDim.x) {
       const size_t at = (size_t)(j >> 6) * P.cap * kWave + (j & 63) * kRun;  // the tile's blocked scratch
-      const uint32_t n = gather_sort_neuron<K, B>(P, t, j, ltd, (uint8_t *)lds, P.cap, P.keys + at, P.keyW + at,
-                                                  ltd ? P.keyPos + at : nullptr);
-      if (threadIdx.x == 0) P.keyCount[j] = n;
-      evSum += n;
+      evSum += gather_sort_neuron<K, B>(P, t, j, ltd, (uint8_t *)lds, P.cap, P.keys + at, P.keyW + at,
+                                        ltd ? P.keyPos + at : nullptr, P.keyCount + j);
     }
     if (!queue) break;
   }
@@ -1807,8 +1929,8 @@ constexpr int kWinPerThread = 12;
 constexpr int kCollectBatches = 4;  // 64-item batches per round of loads (the next round is in flight too)
 
 template <int B, int CH>
-__device__ __attribute__((always_inline)) inline void sort_records(uint32_t t, uint32_t n, uint8_t *lds, uint32_t cap,
-                                                                   uint64_t *out);
+__device__ __attribute__((always_inline)) inline void sort_records(const DevNet &P, uint32_t t, uint32_t j, uint32_t n,
+                                                                   uint32_t nb, uint8_t *lds, uint32_t cap);
 __device__ inline uint64_t *record_runs(const DevNet &P, uint32_t j);
 constexpr uint32_t kSortCap = 768;
 constexpr int kSortChunks = (int)(kSortCap / kWave);
@@ -1984,7 +2106,7 @@ __global__ __launch_bounds__(kCollectThreads) void k_collect(DevNet P, uint32_t 
           if (lane == 0) P.bigList[atomicAdd(P.bigCount, 1u)] = j;
           continue;
         }
-        sort_records<kFusedSortB, kFusedSortChunks>(t, nrec, area, kSortCap, record_runs(P, j));
+        sort_records<kFusedSortB, kFusedSortChunks>(P, t, j, nrec, 0u, area, kSortCap);
       }
     }
   }
@@ -1993,13 +2115,15 @@ __global__ __launch_bounds__(kCollectThreads) void k_collect(DevNet P, uint32_t 
 }
 
 // Orders neuron j's n records (tick << 16 | weight, in live in-list order)
-// in place at out (neuron j's [0][q][0] of the blocked scratch).  Sort key
-// tick << 12 | place: unique, ordered as (arrival time, in-list position).
-// LDS: phase1_lds(cap, B), cap >= n.  Up to CH * 64 records are held in
-// registers; more are read again from out.  Whole wave.
+// in place, its nb bath events among them (at its [0][q][0] of the blocked
+// scratch).  Sort key tick << 12 | place: unique, ordered as (arrival time,
+// in-list position; bath events last).  LDS: phase1_lds(cap, B), cap >= n +
+// nb.  Up to CH * 64 records are held in registers; more are read again from
+// the scratch.  Whole wave.
 template <int B, int CH>
-__device__ __attribute__((always_inline)) inline void sort_records(uint32_t t, uint32_t n, uint8_t *lds, uint32_t cap,
-                                                                   uint64_t *out) {
+__device__ __attribute__((always_inline)) inline void sort_records(const DevNet &P, uint32_t t, uint32_t j, uint32_t n,
+                                                                   uint32_t nb, uint8_t *lds, uint32_t cap) {
+  uint64_t *out = record_runs(P, j);
   constexpr int LOG2B = B == 64 ? 6 : B == 128 ? 7 : B == 256 ? 8 : B == 512 ? 9 : 10;
   uint64_t *sorted = (uint64_t *)lds;
   int16_t *ldsW = (int16_t *)(lds + (size_t)cap * sizeof(uint64_t));
@@ -2035,6 +2159,8 @@ __device__ __attribute__((always_inline)) inline void sort_records(uint32_t t, u
       atomicAdd(&bcnt[key_bucket<B>(rc >> 16, shift)], 1u);
     }
   }
+  uint64_t bk[2];
+  bath_keys<B>(P, dpsnn_asu64((double)t), j, nb, n, shift, bcnt, ldsW, bk);
   wave_sync();
   bucket_scan<B>(bcnt);
   wave_sync();
@@ -2049,8 +2175,9 @@ __device__ __attribute__((always_inline)) inline void sort_records(uint32_t t, u
       sorted[atomicAdd(&bcnt[key_bucket<B>(k >> 12, shift)], 1u)] = k;
     }
   }
+  if (nb) scatter_keys<2, B>(bk, bcnt, sorted, shift);
   wave_sync();  // every record has been read: the runs are rewritten in place
-  rank_in_buckets<B>(sorted, bcnt, n, shift, [&](uint64_t x, uint32_t p) {
+  rank_in_buckets<B>(sorted, bcnt, n + nb, shift, [&](uint64_t x, uint32_t p) {
     out[run_offset(p)] = ((x >> 12) << 16) | (uint16_t)ldsW[x & 0xFFFu];
   });
   wave_sync();
@@ -2073,12 +2200,13 @@ __global__ __launch_bounds__(kWave) void k_sort(DevNet P, uint32_t t) {
   extern __shared__ uint64_t lds[];
   if (P.tDev) t += *P.tDev;
   for (uint32_t j = blockIdx.x; j < P.N; j += gridDim.x) {
-    const uint32_t n = P.keyCount[j];
-    if (n > P.sortCap) {
+    const uint32_t n = P.keyCount[j], nb = bath_count(P, t, j);
+    if (n + nb > P.sortCap) {
       if ((threadIdx.x & 63) == 0) P.bigList[atomicAdd(P.bigCount, 1u)] = j;
       continue;
     }
-    sort_records<B, kSortChunks>(t, n, (uint8_t *)lds, kSortCap, record_runs(P, j));
+    sort_records<B, kSortChunks>(P, t, j, n, nb, (uint8_t *)lds, kSortCap);
+    if (nb && (threadIdx.x & 63) == 0) P.keyCount[j] = n + nb;
   }
 }
 
@@ -2091,8 +2219,9 @@ __global__ __launch_bounds__(kWave) void k_sort_big(DevNet P, uint32_t t) {
   if (blockIdx.x == 0 && threadIdx.x < kXcds) P.winCtr[threadIdx.x * kCtrStride] = 0;  // for the next k_collect
   const uint32_t count = *P.bigCount;
   for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
-    const uint32_t j = P.bigList[i];
-    sort_records<B, kDense>(t, P.keyCount[j], (uint8_t *)lds, P.cap, record_runs(P, j));
+    const uint32_t j = P.bigList[i], n = P.keyCount[j], nb = bath_count(P, t, j);
+    sort_records<B, kDense>(P, t, j, n, nb, (uint8_t *)lds, P.cap);
+    if (nb && (threadIdx.x & 63) == 0) P.keyCount[j] = n + nb;
   }
 }
 
@@ -2132,30 +2261,40 @@ __global__ __launch_bounds__(kBlock) void k_integrate(DevNet P, uint32_t t, ExtV
   if (lane == 0 && ex) atomicAdd(counter_slot(P.counters) + 1, ex);
 }
 
-// k_integrate by integrate_pipe: one workgroup of three waves per tile of 64
-// neurons.
-__global__ __launch_bounds__(kPipeThreads) void k_integrate_pipe(DevNet P, uint32_t t, ExtView X, NextScan S) {
+// Phase 2 of a step with the bath in its records: one lane per neuron ...
+__global__ __launch_bounds__(kBlock) void k_integrate_records(DevNet P, uint32_t t, NextScan S) {
+  __shared__ RecordsLds S2;
+  if (P.tDev) t += *P.tDev;
+  load_exp_table((lds_u64 *)S2.expTab);
+  __syncthreads();
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (blockIdx.x == 0 && threadIdx.x < kXcds) P.workCtr[threadIdx.x * kCtrStride] = 0;  // for the next k_gather
+  if (blockIdx.x == 0 && threadIdx.x == 0 && P.bigCount) *P.bigCount = 0;                 // for the next k_sort
+  const uint32_t j0 = blockIdx.x * kBlock + wave * kWave;
+  const uint32_t m = j0 < P.N ? min((uint32_t)kWave, P.N - j0) : 0u;
+  const uint32_t n = lane < m ? P.keyCount[j0 + lane] : 0u;
+  const size_t at = (size_t)(min(j0, P.N) >> 6) * P.cap * kWave;  // the wave's tile
+  bool f = false;
+  double te = 0.0;
+  integrate_records(P, t, j0, m, P.keys + at, n, (lds_u64 *)S2.stage[wave], (lds_u64 *)S2.expTab, f, te);
+  publish_spikes(P, t + 1, j0 + lane, f, te, S.popCnt, S.count);  // LTP follows in k_ltp
+}
+
+// ... or three waves per tile of 64 neurons.
+__global__ __launch_bounds__(kPipeThreads) void k_integrate_pipe(DevNet P, uint32_t t, NextScan S) {
   __shared__ PipeLds L;
   if (P.tDev) t += *P.tDev;
-  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t lane = threadIdx.x & 63;
   if (blockIdx.x == 0 && threadIdx.x < kXcds) P.workCtr[threadIdx.x * kCtrStride] = 0;  // for the next k_gather
   if (blockIdx.x == 0 && threadIdx.x == 0 && P.bigCount) *P.bigCount = 0;                 // for the next k_sort
   const uint32_t j0 = blockIdx.x * kWave;
   const uint32_t m = min((uint32_t)kWave, P.N - j0);
   const uint32_t n = lane < m ? P.keyCount[j0 + lane] : 0u;
-  const uint64_t *tileK = P.keys + (size_t)blockIdx.x * P.cap * kWave;
   bool f = false;
   double te = 0.0;
-  unsigned long long ex;
-  if (P.drive == DPSNN_DRIVE_REPLAY)
-    ex = integrate_pipe<true>(P, t, X, j0, m, tileK, n, L, f, te);
-  else
-    ex = integrate_pipe<false>(P, t, X, j0, m, tileK, n, L, f, te);
-  if (wave == 2) publish_spikes(P, t + 1, j0 + lane, f, te, S.popCnt, S.count);  // LTP follows in k_ltp
-  if (wave == 0) {
-    for (int o = 32; o > 0; o >>= 1) ex += __shfl_down(ex, o);
-    if (lane == 0 && ex) atomicAdd(counter_slot(P.counters) + 1, ex);
-  }
+  integrate_pipe(P, t, j0, m, P.keys + (size_t)blockIdx.x * P.cap * kWave, n, L, f, te);
+  if (threadIdx.x >= 2 * kWave)
+    publish_spikes(P, t + 1, j0 + lane, f, te, S.popCnt, S.count);  // LTP follows in k_ltp
 }
 
 // The item of global tile g: the last one with tileBegin <= g.
@@ -2194,16 +2333,29 @@ __global__ __launch_bounds__(kWave) void k_batch_gather(const DevNet *nets, cons
     if (j >= P.N) continue;
     const size_t at = (size_t)(u / kWave) * cap * kWave + q * kRun;
     const uint32_t n = gather_sort_neuron<K, B>(P, it.t, j, it.ltd, (uint8_t *)lds, cap, keys + at, keyW + at,
-                                                it.ltd ? keyPos + at : nullptr);
+                                                it.ltd ? keyPos + at : nullptr, keyCount + u);
     if (P.counters != evCtr) {
       if (threadIdx.x == 0 && evSum) atomicAdd(counter_slot(evCtr), evSum);
       evCtr = P.counters;
       evSum = 0;
     }
     evSum += n;
-    if (threadIdx.x == 0) keyCount[u] = n;
   }
   if (threadIdx.x == 0 && evSum) atomicAdd(counter_slot(evCtr), evSum);
+}
+
+// k_bath for the members of global tiles [g0, g1), one wave per tile.
+__global__ __launch_bounds__(kWave) void k_batch_bath(const DevNet *nets, const BatchItem *items, uint32_t count,
+                                                      uint32_t g0) {
+  const uint32_t g = g0 + blockIdx.x;
+  const BatchItem &it = items[batch_item_of(items, count, g)];
+  const DevNet &P = nets[it.net];
+  if (!P.bathT || it.t < kPackT) return;
+  const uint32_t j = (g - it.tileBegin) * kWave + threadIdx.x;
+  if (P.drive == DPSNN_DRIVE_REPLAY)
+    bath_step<true>(P, it.t, it.X, j);
+  else
+    bath_step<false>(P, it.t, it.X, j);
 }
 
 template <int PK>
@@ -2228,7 +2380,12 @@ __global__ __launch_bounds__(kBlock) void k_batch_integrate(const DevNet *nets, 
   bool f = false;
   double te = 0.0;
   unsigned long long ex;
-  if (P.drive == DPSNN_DRIVE_REPLAY)
+  if (P.bathT && it.t >= kPackT) {
+    DevNet Q = P;  // the batch's scratch has its own longest list
+    Q.cap = cap;
+    integrate_records(Q, it.t, j0, m, keys + at, n, (lds_u64 *)S2.stage[wave], (lds_u64 *)S2.expTab, f, te);
+    ex = 0;
+  } else if (P.drive == DPSNN_DRIVE_REPLAY)
     ex = integrate_wave<true, PK>(P, it.t, it.X, j0, m, keys + at, keyW + at, n, (lds_u64 *)S2.stage[wave],
                                   (lds_u64 *)S2.expTab, f, te);
   else
@@ -2497,6 +2654,49 @@ static int upload_window(dpsnn_net *n, int cus) {
   return 0;
 }
 
+static uint32_t round_scratch(uint32_t records) {  // to a whole number of scratch runs
+  return (std::max<uint32_t>(records, 1) + (kRun - 1)) / kRun * kRun;
+}
+
+// The most bath events of a neuron and ms, where a step's bath can be drawn
+// ahead of phase 1 and sorted in there: every sub-population's bath events
+// have one value (a float; DJExt = 0), and the records of a target stay
+// within the 12 bits of the sort key's position.  0: phase 2 draws and merges
+// the bath.  DPSNN_BATH=0 asks for that (tests; the results are the same).
+static uint32_t bath_cap(const dpsnn_net *n) {
+  const Connectome &c = n->con;
+  if (const char *e = std::getenv("DPSNN_BATH"))
+    if (std::atoi(e) == 0) return 0;
+  const char *split = std::getenv("DPSNN_SPLIT"), *fused = std::getenv("DPSNN_FUSED_SORT");
+  if ((split && std::atoi(split) == 0) || (fused && std::atoi(fused) != 0)) return 0;
+  for (uint32_t s = 0; s < n->par.pub.subPopNumber; ++s) {
+    const double *lut = &c.bathLut[size_t(s) * kLutDepth];
+    for (uint32_t i = 0; i < kLutDepth; ++i)
+      if (lut[i] != lut[0] || lut[0] != (double)(float)lut[0]) return 0;
+  }
+  uint32_t cap = 1;
+  for (uint32_t i = 0; i < c.N; ++i) cap = std::max(cap, c.maxExt[i]);
+  return cap <= kBathMax && c.max_in + cap < (1u << 12) - 1 ? cap : 0;
+}
+
+// Bath lists and values on the device, and the scratch's record cap with them.
+static int plan_bath(dpsnn_net *n) {
+  DevNet &P = n->dev;
+  const uint32_t cap = bath_cap(n);
+  if (!cap) return 0;
+  std::vector<float> value(P.nsub);
+  for (uint32_t s = 0; s < P.nsub; ++s) value[s] = (float)n->con.bathLut[size_t(s) * kLutDepth];
+  float *d_value;
+  int rc;
+  if ((rc = dev_alloc(n, &d_value, P.nsub)) || (rc = upload(n, d_value, value.data(), P.nsub)) ||
+      (rc = dev_alloc(n, &P.bathT, (size_t)cap * P.N)) || (rc = dev_alloc(n, &P.bathN, P.N)))
+    return rc;
+  HIP_TRY(hipStreamSynchronize(n->stream));  // `value` ends here
+  P.bathV = d_value;
+  P.cap = round_scratch(n->con.max_in + cap);
+  return 0;
+}
+
 static int build_device(dpsnn_net *n) {
   Connectome &c = n->con;
   const dpsnn_parameters &q = n->par.pub;
@@ -2515,8 +2715,7 @@ static int build_device(dpsnn_net *n) {
   P.nsub = q.subPopNumber;
   P.npc = q.neuronsPerCM;
   P.ncols = q.globCFT;
-  // longest in-list, rounded to a whole number of scratch runs
-  P.cap = (std::max<uint32_t>(c.max_in, 1) + (kRun - 1)) / kRun * kRun;
+  P.cap = round_scratch(c.max_in);  // records of a target (plan_bath adds the bath's)
   // DPSNN_PHASE1_DENSE_MAX lowers the fast path's limit (0: every neuron on
   // the general path), so that tests can compare the two paths
   P.denseMax = kDense * kWave;
@@ -2572,6 +2771,7 @@ static int build_device(dpsnn_net *n) {
     return fail(DPSNN_ERR_CONFIG, "a neuron has %u in-list items; the engine handles up to %u", c.max_in,
                 kMaxInList - 1);
   n->items = c.in_off[N];
+  if ((rc = plan_bath(n))) return rc;
   {
     uint64_t *d_off;
     uint32_t *d_pd;
@@ -2894,16 +3094,21 @@ static bool plastic_at(const dpsnn_net *n, uint32_t t) {
   return n->stdp && t >= q.startPlasticity_ms && t <= q.stopPlasticity_ms;
 }
 
-// Phase 2 of a step with packed records (t >= kPackT): by three waves per
-// tile while the tiles are few.
+// Phase 2 of a step with packed records (t >= kPackT): where they hold the
+// bath, by three waves per tile while the tiles are few.
 static void launch_integrate(const dpsnn_net *n, const DevNet &P, uint32_t t, const ExtView &X, const NextScan &S,
                              hipStream_t stream) {
-  if (n->pipe) {
-    hipLaunchKernelGGL(k_integrate_pipe, dim3(P.NW), dim3(kPipeThreads), 0, stream, P, t, X, S);
-  } else {
-    const uint32_t blocks = (P.N + kBlock - 1) / kBlock;
+  const uint32_t blocks = (P.N + kBlock - 1) / kBlock;
+  if (!P.bathT)
     hipLaunchKernelGGL(k_integrate<1>, dim3(blocks), dim3(kBlock), 0, stream, P, t, X, S);
-  }
+  else if (n->pipe)
+    hipLaunchKernelGGL(k_integrate_pipe, dim3(P.NW), dim3(kPipeThreads), 0, stream, P, t, S);
+  else
+    hipLaunchKernelGGL(k_integrate_records, dim3(blocks), dim3(kBlock), 0, stream, P, t, S);
+}
+// Its bath, ahead of phase 1.
+static void launch_bath(const DevNet &P, uint32_t t, const ExtView &X, hipStream_t stream) {
+  if (P.bathT) hipLaunchKernelGGL(k_bath, dim3(P.NW), dim3(kWave), 0, stream, P, t, X);
 }
 
 // Key scratch of stand-alone steps, blocked by 8 events per neuron:
@@ -2953,6 +3158,9 @@ static int static_scratch_ptr(int device, uint8_t **out) {
 // larger than the array.
 static int static_scratch_view(dpsnn_net *n, DevNet &P) {
   P = n->dev;
+  // the bath stays in phase 2, as the array was sized: a record per in-list item
+  P.bathT = nullptr;
+  P.cap = round_scratch(n->con.max_in);
   const size_t slots = n->split ? size_t(P.NW) * kWave : size_t(n->grid) * kWave;
   auto al = [](size_t b) { return (b + 255) / 256 * 256; };
   const size_t kb = al(slots * P.cap * sizeof(uint64_t)), wb = al(slots * P.cap * sizeof(int16_t)),
@@ -3063,6 +3271,7 @@ static bool window_step(const dpsnn_net *n, const StepPlan &sp) {
 // P (the network's own, or one whose key scratch is a batch's).
 static void launch_window_step(const dpsnn_net *n, const DevNet &P, const StepPlan &sp, hipStream_t stream) {
   const KernelShape &K = kShapes[n->shape];
+  launch_bath(P, sp.t, sp.X, stream);
   hipLaunchKernelGGL(k_collect, dim3(n->winGrid), dim3(kCollectThreads), n->winLds, stream, P, sp.t);
   if (!P.fuseSort)
     hipLaunchKernelGGL(K.sort, dim3(n->sortGrid), dim3(kWave), phase1_lds(kSortCap, K.B), stream, P, sp.t);
@@ -3079,6 +3288,7 @@ static int one_step(dpsnn_net *n, const DevNet &P) {
   if (window_step(n, sp)) {
     launch_window_step(n, P, sp, n->stream);
   } else if (n->split) {
+    if (sp.t >= kPackT) launch_bath(P, sp.t, sp.X, n->stream);
     hipLaunchKernelGGL(K.gather, dim3(n->gatherGrid), dim3(kWave), n->ldsBytes, n->stream, P, sp.t, sp.ltd);
     const uint32_t blocks = (P.N + kBlock - 1) / kBlock;
     if (sp.t >= kPackT)
@@ -3146,6 +3356,7 @@ static int stdp_close(dpsnn_net *n, uint32_t steps, bool failed) {
 // Launches of the graph's step k (t from G.tDev).
 static void launch_graph_step(dpsnn_net *n, const DevNet &G, uint32_t k) {
   const KernelShape &K = kShapes[n->shape];
+  launch_bath(G, k, ExtView{nullptr, nullptr, nullptr}, n->stream);
   if (n->winOn) {
     hipLaunchKernelGGL(k_collect, dim3(n->winGrid), dim3(kCollectThreads), n->winLds, n->stream, G, k);
     if (!G.fuseSort)
@@ -3577,6 +3788,7 @@ uint64_t dpsnn_device_bytes_needed(const dpsnn_net *n) {
   b += 5 * r(8 * N) + r(8 * N);                                // state, Philox counters
   b += r(8 * RS * NW) + r(8 * RS * N);                         // spike history
   b += r(8 * (N + 1)) + r(4 * (items + kWave)) + r(2 * items);  // in-lists
+  if (const uint64_t cap = bath_cap(n)) b += r(4 * q.subPopNumber) + r(8 * cap * N) + r(4 * N);
   if (n->stdp) {
     const uint64_t S = c.S;
     b += r(8 * (N + 1)) + r(2 * S) + r(S) + r(2 * items) + 2 * r(4 * S) + 3 * r(4 * N);
@@ -3995,7 +4207,7 @@ struct dpsnn_batch {
 };
 
 // Scratch the split form may use for one chunk of tiles.
-constexpr size_t kBatchScratchBytes = size_t(5) << 30;  // also holds a 16 x 16-column member in the window form
+constexpr size_t kBatchScratchBytes = size_t(11) << 29;  // also holds a 16 x 16-column member in the window form
 
 namespace {
 
@@ -4037,7 +4249,10 @@ int batch_prepare(dpsnn_batch *b) {
     b->netsCap = count;
   }
   std::vector<DevNet> h(count);
-  for (size_t i = 0; i < count; ++i) h[i] = b->nets[i]->dev;
+  for (size_t i = 0; i < count; ++i) {
+    h[i] = b->nets[i]->dev;
+    if (!b->split) h[i].bathT = nullptr;  // the fused launch merges the bath in phase 2
+  }
   if (count) HIP_TRY(hipMemcpy(b->d_nets, h.data(), sizeof(DevNet) * count, hipMemcpyHostToDevice));
   if (count > b->itemsCap) {
     batch_free_items(b);
@@ -4083,6 +4298,12 @@ int batch_prepare(dpsnn_batch *b) {
   return 0;
 }
 
+// The device copies of the members depend on the form (batch_prepare).
+void batch_set_split(dpsnn_batch *b, bool split) {
+  b->dirty = b->dirty || split != b->split;
+  b->split = split;
+}
+
 uint32_t batch_waves(const dpsnn_batch *b, size_t lds) {
   uint32_t wpc = lds_waves(lds);
   if (b->wavesPerCu) wpc = std::min(wpc, b->wavesPerCu);
@@ -4110,6 +4331,7 @@ int batch_launch(dpsnn_batch *b, int r, uint32_t count, uint32_t tiles, bool pac
           std::min<uint32_t>((g1 - g0) * kWave,
                              (uint32_t)b->cus * std::min(batch_waves(b, lds), resident_waves((const void *)K.batchGather, lds))),
           kXcds);
+      hipLaunchKernelGGL(k_batch_bath, dim3(g1 - g0), dim3(kWave), 0, b->stream, b->d_nets, b->d_items[r], count, g0);
       hipLaunchKernelGGL(K.batchGather, dim3(grid), dim3(kWave), lds, b->stream, b->d_nets, b->d_items[r], count, g0,
                          g1, cap, b->keys, b->keyW, b->keyPos, b->keyCount, b->workCtr);
       const uint32_t blocks = (g1 - g0 + kBlock / kWave - 1) / (kBlock / kWave);
@@ -4358,7 +4580,7 @@ int dpsnn_batch_set_shape(dpsnn_batch *b, const dpsnn_batch_shape *s) {
   if (s->waves_per_cu < 0 || s->waves_per_cu > 16) return fail(DPSNN_ERR_ARG, "waves_per_cu must be in 0..16");
   b->shape = i;
   b->wavesPerCu = (uint32_t)s->waves_per_cu;
-  b->split = s->split != 0;
+  batch_set_split(b, s->split != 0);
   return 0;
 }
 
@@ -4394,7 +4616,7 @@ int dpsnn_batch_tune(dpsnn_batch *b, uint32_t trial_steps, dpsnn_batch_shape *ch
       for (uint32_t w : {0u, std::max<uint32_t>(1, top / 2)}) {
         b->shape = i;
         b->wavesPerCu = w;
-        b->split = split != 0;
+        batch_set_split(b, split != 0);
         HIP_TRY(hipStreamSynchronize(b->stream));
         b->profile = true;
         b->evUsed = 0;
@@ -4414,7 +4636,7 @@ int dpsnn_batch_tune(dpsnn_batch *b, uint32_t trial_steps, dpsnn_batch_shape *ch
     }
   b->shape = bestShape;
   b->wavesPerCu = bestWaves;
-  b->split = bestSplit;
+  batch_set_split(b, bestSplit);
   b->profile = wasProfiling;
   if (chosen) {
     chosen->chunks = kShapes[bestShape].K;
