@@ -2417,6 +2417,27 @@ __global__ __launch_bounds__(kWaveLTP) void k_batch_ltp(const DevNet *nets, cons
 // The first step of a graph replay, set before it.
 __global__ void k_set_t(uint32_t *t, uint32_t v) { *t = v; }
 
+// The state after step t - 1 (slot t holds its spikes) into pinned host memory:
+// v, c, Tr, Te [N] each, then a byte per neuron that fired.
+__global__ __launch_bounds__(kBlock) void k_read_state(DevNet P, uint32_t t, double *out) {
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= P.N) return;
+  out[i] = P.v[i];
+  out[(size_t)P.N + i] = P.c[i];
+  out[2 * (size_t)P.N + i] = P.Tr[i];
+  out[3 * (size_t)P.N + i] = P.Te[i];
+  const uint64_t w = P.bits[(size_t)(t & (P.RS - 1)) * P.NW + (i >> 6)];
+  ((uint8_t *)(out + 4 * (size_t)P.N))[i] = (uint8_t)((w >> (i & 63)) & 1ull);
+}
+
+// The sums of the first kReadCounters counters into pinned host memory.
+constexpr uint32_t kReadCounters = 4;
+__global__ void k_read_counters(const unsigned long long *counters, unsigned long long *out) {
+  unsigned long long sum = 0;
+  for (uint32_t k = 0; k < kCounterSlots; ++k) sum += counters[k * kCounterStride + threadIdx.x];
+  out[threadIdx.x] = sum;
+}
+
 // Fills n doubles with v.
 __global__ void k_fill_f64(double *p, double v, uint64_t n) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
@@ -2559,6 +2580,12 @@ struct dpsnn_net {
   bool graphs = true;        // DPSNN_GRAPH=0: plain launches only
   uint64_t graphSteps = 0;   // steps replayed from the graph so far
   bool collect = false;  // raster / rates are being produced
+  // pinned host memory of read-backs, allocated at the first one; readMu: two
+  // threads may read one network's state or counters at a time
+  std::mutex readMu;
+  double *h_state = nullptr;                 // k_read_state's
+  unsigned long long *h_counters = nullptr;  // k_read_counters'
+  uint8_t *h_drain = nullptr;                // kDrainBytes
 };
 
 template <class T>
@@ -2591,6 +2618,11 @@ static void free_all(dpsnn_net *n) {
     if (s.done) hipEventDestroy(s.done);
     s = ExtSlot{};
   }
+  for (void *p : {(void *)n->h_state, (void *)n->h_counters, (void *)n->h_drain})
+    if (p) (void)hipHostFree(p);
+  n->h_state = nullptr;
+  n->h_counters = nullptr;
+  n->h_drain = nullptr;
   for (auto &e : n->profEv) {
     hipEventDestroy(e.a);
     hipEventDestroy(e.b);
@@ -2919,6 +2951,39 @@ static int ensure_ext_cap(ExtSlot &s, size_t need) {
   return 0;
 }
 
+// Device-to-host copies gathered in pinned memory: a copy into pageable memory
+// costs the caller 30 us and a wait each.  add() queues one (a piece that does
+// not fit goes straight to its place); fetch() waits for the stream and moves
+// the pieces to theirs.
+constexpr size_t kDrainBytes = size_t(1) << 18;
+struct PinnedCopies {
+  dpsnn_net *n;
+  size_t used = 0;
+  struct Piece {
+    void *to;
+    size_t at, bytes;
+  };
+  std::vector<Piece> pieces;
+  int add(void *to, const void *from, size_t bytes) {
+    if (!n->h_drain) HIP_TRY(hipHostMalloc((void **)&n->h_drain, kDrainBytes, 0));
+    if (used + bytes > kDrainBytes) {
+      HIP_TRY(hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToHost, n->stream));
+      return 0;
+    }
+    HIP_TRY(hipMemcpyAsync(n->h_drain + used, from, bytes, hipMemcpyDeviceToHost, n->stream));
+    pieces.push_back({to, used, bytes});
+    used += (bytes + 63) / 64 * 64;
+    return 0;
+  }
+  int fetch() {
+    HIP_TRY(hipStreamSynchronize(n->stream));
+    for (const Piece &p : pieces) std::memcpy(p.to, n->h_drain + p.at, p.bytes);
+    pieces.clear();
+    used = 0;
+    return 0;
+  }
+};
+
 // Copies the pending raster / rates out of device memory and writes files.
 static int drain(dpsnn_net *n) {
   if (n->opt.keep_spikes && n->aheadMs != UINT32_MAX && n->aheadMs + 1 == n->t) {
@@ -2930,28 +2995,25 @@ static int drain(dpsnn_net *n) {
   const DevNet &P = n->dev;
   const size_t popPer = size_t(P.ncols) * P.nsub;
   const uint32_t steps = n->pendingSteps;
+  PinnedCopies copies{n};
+  int rc;
   n->h_pop.resize(popPer * steps);
-  HIP_TRY(hipMemcpyAsync(n->h_pop.data(), n->d_popCnt, sizeof(uint32_t) * popPer * steps,
-                         hipMemcpyDeviceToHost, n->stream));
+  if ((rc = copies.add(n->h_pop.data(), n->d_popCnt, sizeof(uint32_t) * popPer * steps))) return rc;
   uint32_t total = 0;
   if (n->wantRaster) {
     n->h_steps.resize(steps);
-    HIP_TRY(hipMemcpyAsync(n->h_steps.data(), n->d_stepCount, sizeof(uint32_t) * steps,
-                           hipMemcpyDeviceToHost, n->stream));
-    HIP_TRY(hipMemcpyAsync(&total, n->d_rasterCount, sizeof(uint32_t), hipMemcpyDeviceToHost, n->stream));
-    HIP_TRY(hipStreamSynchronize(n->stream));
+    if ((rc = copies.add(n->h_steps.data(), n->d_stepCount, sizeof(uint32_t) * steps)) ||
+        (rc = copies.add(&total, n->d_rasterCount, sizeof(uint32_t))) || (rc = copies.fetch()))
+      return rc;
     n->h_ids.resize(total);
     n->h_te.resize(total);
-    if (total) {
-      HIP_TRY(hipMemcpyAsync(n->h_ids.data(), n->d_rasterIds, sizeof(uint32_t) * total,
-                             hipMemcpyDeviceToHost, n->stream));
-      HIP_TRY(hipMemcpyAsync(n->h_te.data(), n->d_rasterTe, sizeof(double) * total,
-                             hipMemcpyDeviceToHost, n->stream));
-    }
+    if (total && ((rc = copies.add(n->h_ids.data(), n->d_rasterIds, sizeof(uint32_t) * total)) ||
+                  (rc = copies.add(n->h_te.data(), n->d_rasterTe, sizeof(double) * total))))
+      return rc;
     HIP_TRY(hipMemsetAsync(n->d_rasterCount, 0, sizeof(uint32_t), n->stream));
   }
   HIP_TRY(hipMemsetAsync(n->d_popCnt, 0, sizeof(uint32_t) * popPer * steps, n->stream));
-  HIP_TRY(hipStreamSynchronize(n->stream));
+  if ((rc = copies.fetch())) return rc;
   uint32_t pos = 0;
   for (uint32_t k = 0; k < steps; ++k) {
     const uint32_t cnt = n->wantRaster ? n->h_steps[k] : 0;
@@ -3902,9 +3964,30 @@ int dpsnn_sync(dpsnn_net *n) {
 uint32_t dpsnn_now_ms(const dpsnn_net *n) { return n ? n->t : 0; }
 uint32_t dpsnn_total_ms(const dpsnn_net *n) { return n ? n->par.pub.totalSimTime_ms : 0; }
 
+// Up to this many neurons one kernel writes the state to pinned memory: five
+// copies into pageable memory took 30 us each whatever their size.  A step and
+// its read-backs: one column 206 -> 143 us, 2x2 with its spikes 351 -> 259.
+// Above, a ms takes 400 us and more; the line bounds the pinned memory of a
+// network (4.3 MB).
+static constexpr size_t kStateDirect = size_t(1) << 17;
+
 int dpsnn_get_state(dpsnn_net *n, double *v, double *c, double *Tr, double *Te, uint8_t *fired) {
   if (!n) return fail(DPSNN_ERR_ARG, "null network");
   const size_t N = n->dev.N;
+  if (n->uploaded && N <= kStateDirect) {
+    std::lock_guard<std::mutex> lk(n->readMu);
+    HIP_TRY(hipSetDevice(n->opt.device));
+    if (!n->h_state) HIP_TRY(hipHostMalloc((void **)&n->h_state, N * 33 + 8, 0));
+    hipLaunchKernelGGL(k_read_state, dim3((uint32_t)((N + kBlock - 1) / kBlock)), dim3(kBlock), 0, n->stream, n->dev,
+                       n->t, n->h_state);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(n->stream));
+    double *to[4] = {v, c, Tr, Te};
+    for (int i = 0; i < 4; ++i)
+      if (to[i]) std::memcpy(to[i], n->h_state + N * (size_t)i, N * 8);
+    if (fired) std::memcpy(fired, n->h_state + 4 * N, N);
+    return 0;
+  }
   HIP_TRY(hipStreamSynchronize(n->stream));
   if (v) HIP_TRY(hipMemcpy(v, n->dev.v, N * 8, hipMemcpyDeviceToHost));
   if (c) HIP_TRY(hipMemcpy(c, n->dev.c, N * 8, hipMemcpyDeviceToHost));
@@ -3952,11 +4035,14 @@ int dpsnn_get_synapses(dpsnn_net *n, uint32_t *pre, uint32_t *post, uint8_t *del
 int dpsnn_write_synapse_dump(dpsnn_net *n, const char *path);
 int dpsnn_get_stats(dpsnn_net *n, dpsnn_stats *out) {
   if (!n || !out) return fail(DPSNN_ERR_ARG, "null argument");
-  unsigned long long slots[kCounterSlots * kCounterStride], cnt[4] = {0, 0, 0, 0};
+  if (!n->uploaded) return fail(DPSNN_ERR_ARG, "network not uploaded (dpsnn_upload)");
+  std::lock_guard<std::mutex> lk(n->readMu);
+  HIP_TRY(hipSetDevice(n->opt.device));
+  if (!n->h_counters) HIP_TRY(hipHostMalloc((void **)&n->h_counters, kReadCounters * sizeof(unsigned long long), 0));
+  hipLaunchKernelGGL(k_read_counters, dim3(1), dim3(kReadCounters), 0, n->stream, n->dev.counters, n->h_counters);
+  HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(n->stream));
-  HIP_TRY(hipMemcpy(slots, n->dev.counters, sizeof slots, hipMemcpyDeviceToHost));
-  for (uint32_t k = 0; k < kCounterSlots; ++k)
-    for (int i = 0; i < 4; ++i) cnt[i] += slots[k * kCounterStride + i];
+  const unsigned long long *cnt = n->h_counters;
   out->steps = n->t;
   out->synaptic_events = cnt[0];
   out->external_events = cnt[1];
