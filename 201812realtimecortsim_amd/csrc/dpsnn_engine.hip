@@ -1880,11 +1880,25 @@ __global__ __launch_bounds__(kWave) void k_gather(DevNet P, uint32_t t, int ltd)
 // place, as phase 2 reads them.
 // ---------------------------------------------------------------------------
 constexpr int kCollectThreads = kWindowWaves * kWave;
-constexpr uint32_t kWindowMinNeurons = 1u << 16;  // the window form by default from this size
-// Targets per unit: enough items per pass to amortise the pass's window
-// load, units small enough for a short queue tail (1250-neuron columns: 4
-// units of 313; measured best on grids of 8x8, 12x12 and 24x24 columns)
+// The window form by default from this size.  k_gather is bound by the L1
+// misses of its emission-time loads, one line per event (68% of its cycles;
+// more waves a CU don't help), which the window's LDS saves; below, k_gather
+// deals its targets out in the fixed order and the window's passes cost more
+// than its events (ms per step, gather and window: 5,000 neurons 0.070 and
+// 0.080, 10,000 neurons 0.091 and 0.103, 12,000 0.144 and 0.151, 12,500 0.106
+// and 0.091, 18,252 0.127 and 0.110, 31,250 0.49 and 0.38, 45,000 0.53 and
+// 0.39).
+constexpr uint32_t kWindowMinNeurons = 12288;
+// In a batch a window-form member steps on launches of its own: from this
+// size on they fill the device.
+constexpr uint32_t kBatchWindowMin = 1u << 16;
+// Targets per unit, at most: enough items per pass to amortise the pass's
+// window load, units small enough for a short queue tail (1250-neuron columns:
+// 4 units of 313; measured best on grids of 8x8, 12x12 and 24x24 columns).
+// Small networks: as many units as fit one per CU (ms per step with 108, 216,
+// 252 and 288 units of 45,000 neurons: 0.49, 0.41, 0.39 and 0.45).
 constexpr uint32_t kWindowUnitTargets = 320;
+constexpr uint32_t kWindowUnits = 256;
 constexpr uint32_t kWindowMaxEntries = 12 * 1024;  // window entries: kWinPerThread per thread of k_collect
 
 // Block-wide work queue: the next unit for the whole workgroup (one unit
@@ -2430,6 +2444,57 @@ __global__ __launch_bounds__(kBlock) void k_read_state(DevNet P, uint32_t t, dou
   ((uint8_t *)(out + 4 * (size_t)P.N))[i] = (uint8_t)((w >> (i & 63)) & 1ull);
 }
 
+// The window layout's items and chunk descriptors from the in-lists (the
+// host's build_window with fill; there they cost the host 50 ms and their
+// upload for 45,000 neurons of 1,250 items, here a launch of 0.3 ms).  One
+// workgroup per unit, wave w its targets q = w, w + kWindowWaves, ...: the
+// first item of each run of one delay leaves its place in start[], every item
+// finds its own from it, and base[] moves on by the run's chunks.
+constexpr uint32_t kMaxPasses = 256;  // run delays are bytes
+__global__ __launch_bounds__(kCollectThreads) void k_window_fill(DevNet P, uint32_t *item, uint16_t *desc) {
+  __shared__ uint32_t startOf[kWindowWaves][kMaxPasses], baseOf[kWindowWaves][kMaxPasses];
+  constexpr uint32_t C = kWindowChunk;
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63, u = blockIdx.x;
+  uint32_t *start = startOf[wave], *base = baseOf[wave];
+  const uint32_t col = u / P.winUnitsPerCol, part = u - col * P.winUnitsPerCol;
+  const uint32_t j0 = col * P.npc + part * P.winUnit;
+  const uint32_t m = min(P.winUnit, (col + 1) * P.npc - j0);
+  const int32_t *cols = P.winCols + (size_t)col * P.winSlots;
+  for (uint32_t d = lane; d < P.winPasses; d += kWave)
+    base[d] = (uint32_t)P.winChunk[((size_t)u * P.winPasses + (P.winPasses - 1 - d)) * kWindowWaves + wave];
+  for (uint32_t q = wave; q < m; q += kWindowWaves) {
+    const uint64_t beg = P.inOff[j0 + q];
+    const uint32_t len = (uint32_t)(P.inOff[j0 + q + 1] - beg);
+    const uint32_t *in = P.inPD + beg;
+    for (uint32_t i = lane; i < len; i += kWave) {
+      const uint32_t d = in[i] >> 24;
+      if (i == 0 || in[i - 1] >> 24 != d) start[d] = i;
+    }
+    wave_sync();
+    for (uint32_t i = lane; i < len; i += kWave) {
+      const uint32_t d = in[i] >> 24, src = in[i] & 0xFFFFFFu, sc = src / P.npc, off = i - start[d];
+      uint32_t lo = 0, hi = P.winSlots;  // the slot of column sc: cols ascends, then -1
+      while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) / 2;
+        if ((uint32_t)cols[mid] <= sc) lo = mid;  // -1: the largest
+        else hi = mid;
+      }
+      const size_t ch = (size_t)base[d] + off / C;
+      item[ch * C + off % C] = (lo * P.npc + (src - sc * P.npc)) << 16 | (uint16_t)P.inW[beg + i];
+      if (off % C == 0) desc[ch] = (uint16_t)(q | (off == 0 ? kWindowFirst : 0u));
+    }
+    wave_sync();
+    for (uint32_t i = lane; i < len; i += kWave) {
+      const uint32_t d = in[i] >> 24;
+      if (i + 1 < len && in[i + 1] >> 24 == d) continue;
+      const uint32_t off = i - start[d], ch = base[d] + off / C;  // the run's last item
+      for (uint32_t x = off % C + 1; x < C; ++x) item[(size_t)ch * C + x] = P.winSlots * P.npc << 16;
+      base[d] = ch + 1;
+    }
+    wave_sync();
+  }
+}
+
 // The sums of the first kReadCounters counters into pinned host memory.
 constexpr uint32_t kReadCounters = 4;
 __global__ void k_read_counters(const unsigned long long *counters, unsigned long long *out) {
@@ -2660,8 +2725,8 @@ static int upload_window(dpsnn_net *n, int cus) {
   uint64_t *d_chunk;
   int32_t *d_cols;
   int rc;
-  if ((rc = dev_alloc(n, &d_item, L.item.size())) || (rc = upload(n, d_item, L.item.data(), L.item.size())) ||
-      (rc = dev_alloc(n, &d_desc, L.desc.size())) || (rc = upload(n, d_desc, L.desc.data(), L.desc.size())) ||
+  if (L.passes > kMaxPasses) return fail(DPSNN_ERR_CONFIG, "%u run delays", L.passes);
+  if ((rc = dev_alloc(n, &d_item, L.items())) || (rc = dev_alloc(n, &d_desc, L.chunks())) ||
       (rc = dev_alloc(n, &d_chunk, L.chunk.size())) || (rc = upload(n, d_chunk, L.chunk.data(), L.chunk.size())) ||
       (rc = dev_alloc(n, &d_cols, L.cols.size())) || (rc = upload(n, d_cols, L.cols.data(), L.cols.size())) ||
       (rc = dev_alloc(n, &P.winCtr, kXcds * kCtrStride)) || (rc = dev_alloc(n, &P.bigList, P.N)) ||
@@ -2669,10 +2734,12 @@ static int upload_window(dpsnn_net *n, int cus) {
     return rc;
   HIP_TRY(hipMemsetAsync(P.winCtr, 0, sizeof(uint32_t) * kXcds * kCtrStride, n->stream));
   HIP_TRY(hipMemsetAsync(P.bigCount, 0, sizeof(uint32_t), n->stream));
-  HIP_TRY(hipStreamSynchronize(n->stream));  // the host staging is dropped after upload
   P.winItem = d_item; P.winDesc = d_desc; P.winChunk = d_chunk; P.winCols = d_cols;
   P.winSlots = L.slots; P.winPasses = L.passes; P.winUnit = L.unit; P.winUnitsPerCol = L.unitsPerCol;
   P.winUnits = L.units;
+  hipLaunchKernelGGL(k_window_fill, dim3(L.units), dim3(kCollectThreads), 0, n->stream, P, d_item, d_desc);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipStreamSynchronize(n->stream));  // the host staging is dropped after upload
   // DPSNN_SORT_CAP lowers k_sort's limit, so that tests send targets through
   // k_sort_big
   P.sortCap = kSortCap;
@@ -3813,10 +3880,13 @@ int dpsnn_prepare(const char *inidir, const dpsnn_options *opt, dpsnn_net **out)
       // DPSNN_WINDOW_UNITS: units wanted per step instead (tuning; results do
       // not change)
       const char *ue = getenv("DPSNN_WINDOW_UNITS");
+      const uint32_t wanted = std::max<uint32_t>((q.neuronsPerCM + kWindowUnitTargets - 1) / kWindowUnitTargets,
+                                                 kWindowUnits / std::max(q.globCFT, 1u));
       const uint32_t unitsPerCol =
           ue && atoi(ue) > 0 ? std::max<uint32_t>(1, ((uint32_t)atoi(ue) + q.globCFT - 1) / q.globCFT)
-                             : std::max<uint32_t>(1, (q.neuronsPerCM + kWindowUnitTargets - 1) / kWindowUnitTargets);
-      build_window(n->par, n->con, unitsPerCol, kWindowMaxEntries, n->window, n->opt.host_threads);
+                             : std::max<uint32_t>(1, wanted);
+      build_window(n->par, n->con, unitsPerCol, kWindowMaxEntries, n->window, n->opt.host_threads,
+                   /*fill=*/false);
     }
   }
   if (n->opt.drive == DPSNN_DRIVE_REPLAY) n->replay.init(n->con, &n->rng);
@@ -3867,7 +3937,7 @@ uint64_t dpsnn_device_bytes_needed(const dpsnn_net *n) {
   if (n->opt.drive == DPSNN_DRIVE_REPLAY) b += kExtRing * r(4 * (N + 1));
   const WindowLayout &L = n->window;
   if (L.ok)
-    b += r(4 * L.item.size()) + r(2 * L.desc.size()) + r(8 * L.chunk.size()) + r(4 * L.cols.size()) +
+    b += r(4 * L.items()) + r(2 * L.chunks()) + r(8 * L.chunk.size()) + r(4 * L.cols.size()) +
          r(4 * kXcds * kCtrStride) + r(4 * N) + r(4);
   return b;
 }
@@ -4503,7 +4573,7 @@ int batch_one_step(dpsnn_batch *b, bool *any) {
     if ((rc = pre_step(n, sp))) return rc;
     // a member whose step runs in the window form, and whose tiles fit the
     // batch's key scratch, steps on its own launches (below)
-    if (window_step(n, sp) && (size_t)n->dev.NW * kWave <= b->scratchSlots) {
+    if (n->dev.N >= kBatchWindowMin && window_step(n, sp) && (size_t)n->dev.NW * kWave <= b->scratchSlots) {
       b->windowed.push_back((uint32_t)i);
       continue;
     }

@@ -1238,7 +1238,7 @@ void build_delivery(const Params &p, Connectome &c, bool with_incoming, unsigned
 // order, i.e. run delay descending, then source ascending.
 // --------------------------------------------------------------------------
 void build_window(const Params &p, const Connectome &c, uint32_t unitsPerCol, uint32_t maxEntries,
-                  WindowLayout &L, unsigned threads) {
+                  WindowLayout &L, unsigned threads, bool fill) {
   L = WindowLayout{};
   const uint32_t N = c.N, npc = p.pub.neuronsPerCM, ncols = p.pub.globCFT;
   if (N == 0 || c.in_off.size() != size_t(N) + 1 || c.in_pre_d.size() != c.in_off[N]) {
@@ -1265,10 +1265,14 @@ void build_window(const Params &p, const Connectome &c, uint32_t unitsPerCol, ui
   std::vector<uint32_t> maxD(ncols, 0);
   parallel(ncols, [&](uint32_t col) {
     std::vector<uint8_t> seen(ncols, 0);
-    uint32_t md = 0;
+    uint32_t md = 0, from = 0, span = 0;  // a run's sources ascend: mostly the last one's column again
     for (uint64_t k = c.in_off[uint64_t(col) * npc]; k < c.in_off[uint64_t(col + 1) * npc]; ++k) {
-      const uint32_t pd = c.in_pre_d[k];
-      seen[(pd & 0xFFFFFFu) / npc] = 1;
+      const uint32_t pd = c.in_pre_d[k], src = pd & 0xFFFFFFu;
+      if (src - from >= span) {
+        seen[src / npc] = 1;
+        from = src / npc * npc;
+        span = npc;
+      }
       md = std::max(md, pd >> 24);
     }
     for (uint32_t s = 0; s < ncols; ++s)
@@ -1332,6 +1336,8 @@ void build_window(const Params &p, const Connectome &c, uint32_t unitsPerCol, ui
     L.chunk.clear();
     return;
   }
+  L.ok = true;
+  if (!fill) return;
   L.item.assign(L.chunk[streams] * C, (uint32_t)(slots * npc) << 16);
   L.desc.assign(L.chunk[streams], 0);
   parallel(L.units, [&](uint32_t u) {
@@ -1362,7 +1368,6 @@ void build_window(const Params &p, const Connectome &c, uint32_t unitsPerCol, ui
       }
     }
   });
-  L.ok = true;
 }
 
 // --------------------------------------------------------------------------

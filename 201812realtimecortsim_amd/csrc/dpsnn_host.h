@@ -163,13 +163,16 @@ struct WindowLayout {
   std::vector<uint32_t> item;
   std::vector<uint16_t> desc;
   std::vector<uint64_t> chunk;
+  uint64_t chunks() const { return chunk.empty() ? 0 : chunk.back(); }
+  uint64_t items() const { return chunks() * kWindowChunk; }
 };
 // Builds the layout from c's in-lists with at most `maxSlots` stencil slots
 // (window entries slots * npc + 1 <= maxEntries) and units of
 // ceil(npc / unitsPerCol) targets; sets ok = false (and why) when the
-// connectome does not fit.
+// connectome does not fit.  Without `fill`, item and desc stay empty: the
+// engine writes them on the device, from the in-lists there.
 void build_window(const Params &p, const Connectome &c, uint32_t unitsPerCol, uint32_t maxEntries,
-                  WindowLayout &L, unsigned threads = 0);
+                  WindowLayout &L, unsigned threads = 0, bool fill = true);
 
 // Host-side replay of the external Poisson drive (DPSNN_neuron_sim.c:
 // 604-640, :844-865): the reference's ran3 draws in neuron order, step by

@@ -100,3 +100,43 @@ def test_grid24_small_columns_bit_exact_vs_oracle(pkg, oracle, tmp_path, monkeyp
     print(f"window={window} fused={fused}: 24x24 x 40 neurons, 80 ms vs oracle", flush=True)
     st = _trace_vs_oracle(pkg, oracle, cfg, 80, 8)
     assert st["neurons"] == 576 * 40 and st["spikes"] > 0 and st["synaptic_events"] > 0
+
+
+# either side of the size from which the window form is the default (12,288
+# neurons): 49 columns of 250, 36 of 347 and 961 of 13
+@pytest.mark.parametrize("counts,side,form", [((100, 100, 50), 7, 0), ((139, 139, 69), 6, 1), ((5, 5, 3), 31, 1)])
+@pytest.mark.parametrize("units", [None, "1", "200"])
+def test_default_form_and_its_layout(pkg, tmp_path, monkeypatch, counts, side, form, units):
+    """The default form, whose layout the device fills, against the gather
+    form; a member of a batch of this size stays in the batch's launches."""
+    cfg = _columns(tmp_path, pkg, "d", counts, nu_ext=4.0)
+    pkg.apply_env(pkg.config_dir("c0"), env_CFX=side, env_CFY=side, env_totalSimTime_ms=60)
+    if units:
+        monkeypatch.setenv("DPSNN_WINDOW_UNITS", units)
+    print(f"{side}x{side} columns of {counts}, window units {units}: default form vs gather", flush=True)
+    states, events = [], []
+    for how in ("default", "gather", "batch"):
+        if how == "gather":
+            monkeypatch.setenv("DPSNN_WINDOW", "0")
+        else:
+            monkeypatch.delenv("DPSNN_WINDOW", raising=False)
+        with pkg.Network(cfg) as net:
+            if how == "batch":
+                with pkg.Batch() as b:
+                    b.add(net)
+                    b.step(60)
+                    b.sync()
+                    states.append(net.state())
+                    events.append(net.stats()["synaptic_events"])
+                    b.remove(net)
+                continue
+            net.step(45)
+            net.step(15)
+            states.append(net.state())
+            st = net.stats()
+            events.append(st["synaptic_events"])
+            assert st["window_form"] == (form if how == "default" else 0)
+    assert events[0] == events[1] == events[2] > 0
+    for other in states[1:]:
+        for k in ("v", "c", "Tr", "Te"):
+            assert np.array_equal(states[0][k].view(np.uint64), other[k].view(np.uint64)), k
