@@ -1512,10 +1512,14 @@ __device__ __attribute__((always_inline)) inline void scatter_keys(const uint64_
     if (key[k] != kNoKey) sorted[atomicAdd(&bcnt[key_bucket<B>(key[k] >> 12, shift)], 1u)] = key[k];
 }
 
+// Keys that rank_in_buckets reads at a time, and the padding after the sort
+// buffer that lets it read past the last bucket's end.
+constexpr uint32_t kRankReads = 6;
+
 // LDS of one phase-1 wave: sort buffer (u64) and weights by position (i16)
-// for the longest in-list, then the bucket counters.
+// for the longest in-list, then the bucket counters after a zero.
 __host__ __device__ inline size_t phase1_lds(uint32_t cap, int B) {
-  return (size_t)cap * sizeof(uint64_t) + (size_t)cap * sizeof(int16_t) + (size_t)(B + 1) * sizeof(uint32_t);
+  return (size_t)(cap + kRankReads) * sizeof(uint64_t) + (size_t)cap * sizeof(int16_t) + (size_t)(B + 2) * sizeof(uint32_t);
 }
 
 // Offset of event p of a neuron in the tile's blocked scratch, from the
@@ -1546,23 +1550,35 @@ __device__ __attribute__((always_inline)) inline void bucket_scan(uint32_t *bcnt
 // The n keys in sorted[] are scattered into their buckets (bcnt[b] = end of
 // bucket b).  Within a bucket each key's place is its rank (keys are
 // unique): the count of the bucket's smaller keys.  Calls put(key, place)
-// once per key.  Lanes take the keys in bucket order, so
-// lanes of one bucket read the same words together; the reads are
-// independent of each other.  Whole wave.
+// once per key.  Lanes take the keys in bucket order, so lanes of one bucket
+// read the same words together.  The kRankReads independent reads of a round
+// may pass the bucket's end: the keys there are larger (a later bucket, or
+// the padding).  The sorts are bound by their instructions and LDS reads, and
+// most are here (a bucket holds 4-14 keys, most of them one spike time):
+// rounds of 4 with the remainder one key at a time took 189 us at 80,000
+// neurons (k_sort, now 180), 1,206 for a batch of 150,000 (k_batch_gather,
+// now 1,157).  Reads of 4 and 8: 180 and 182, 1,163 and 1,152.  bcnt[-1] is a
+// word of its own.  Whole wave.
 template <int B, class Put>
-__device__ __attribute__((always_inline)) inline void rank_in_buckets(const uint64_t *sorted, const uint32_t *bcnt,
+__device__ __attribute__((always_inline)) inline void rank_in_buckets(uint64_t *sorted, uint32_t *bcnt,
                                                                       uint32_t n, int shift, Put &&put) {
-  for (uint32_t i = threadIdx.x & 63; i < n; i += kWave) {
+  const uint32_t lane = threadIdx.x & 63;
+  if (lane < kRankReads) sorted[n + lane] = kNoKey;
+  if (lane == 0) bcnt[-1] = 0;
+  wave_sync();
+  for (uint32_t i = lane; i < n; i += kWave) {
     const uint64_t x = sorted[i];
-    const uint32_t b = key_bucket<B>(x >> 12, shift);
-    const uint32_t lo = b ? bcnt[b - 1] : 0u, hi = bcnt[b];
-    uint32_t r = 0, y = lo;
-    for (; y + 4 <= hi; y += 4) {  // four independent reads per round
-      const uint64_t a0 = sorted[y], a1 = sorted[y + 1], a2 = sorted[y + 2], a3 = sorted[y + 3];
-      r += (a0 < x ? 1u : 0u) + (a1 < x ? 1u : 0u) + (a2 < x ? 1u : 0u) + (a3 < x ? 1u : 0u);
+    const uint32_t b = key_bucket<B>(x, shift + 12);
+    const uint32_t lo = (bcnt - 1)[b], hi = bcnt[b];
+    uint32_t r = lo;
+    for (uint32_t y = lo; y < hi; y += kRankReads) {
+      uint64_t a[kRankReads];
+#pragma unroll
+      for (uint32_t k = 0; k < kRankReads; ++k) a[k] = sorted[y + k];
+#pragma unroll
+      for (uint32_t k = 0; k < kRankReads; ++k) r += a[k] < x ? 1u : 0u;
     }
-    for (; y < hi; ++y) r += sorted[y] < x ? 1u : 0u;
-    put(x, lo + r);
+    put(x, r);
   }
 }
 
@@ -1611,8 +1627,8 @@ __device__ __attribute__((always_inline)) inline uint32_t gather_sort_neuron(con
   static_assert(B % kWave == 0, "bucket count must be a multiple of 64");
   constexpr int LOG2B = B == 64 ? 6 : B == 128 ? 7 : B == 256 ? 8 : B == 512 ? 9 : 10;
   uint64_t *sorted = (uint64_t *)lds;
-  int16_t *ldsW = (int16_t *)(lds + (size_t)cap * sizeof(uint64_t));
-  uint32_t *bcnt = (uint32_t *)(lds + (size_t)cap * (sizeof(uint64_t) + sizeof(int16_t)));
+  int16_t *ldsW = (int16_t *)(sorted + cap + kRankReads);
+  uint32_t *bcnt = (uint32_t *)(ldsW + cap) + 1;
   const uint32_t lane = threadIdx.x & 63;
   const uint64_t tBits = dpsnn_asu64((double)t);
   const double tF = (double)t;
@@ -2140,8 +2156,8 @@ __device__ __attribute__((always_inline)) inline void sort_records(const DevNet 
   uint64_t *out = record_runs(P, j);
   constexpr int LOG2B = B == 64 ? 6 : B == 128 ? 7 : B == 256 ? 8 : B == 512 ? 9 : 10;
   uint64_t *sorted = (uint64_t *)lds;
-  int16_t *ldsW = (int16_t *)(lds + (size_t)cap * sizeof(uint64_t));
-  uint32_t *bcnt = (uint32_t *)(lds + (size_t)cap * (sizeof(uint64_t) + sizeof(int16_t)));
+  int16_t *ldsW = (int16_t *)(sorted + cap + kRankReads);
+  uint32_t *bcnt = (uint32_t *)(ldsW + cap) + 1;
   const uint32_t lane = threadIdx.x & 63;
   const int shift = 52 - LOG2B - (31 - __clz((int)t));
   for (uint32_t b = lane; b <= (uint32_t)B; b += kWave) bcnt[b] = 0;
