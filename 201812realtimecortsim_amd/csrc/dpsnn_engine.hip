@@ -1908,13 +1908,28 @@ constexpr uint32_t kWindowMinNeurons = 12288;
 // In a batch a window-form member steps on launches of its own: from this
 // size on they fill the device.
 constexpr uint32_t kBatchWindowMin = 1u << 16;
-// Targets per unit, at most: enough items per pass to amortise the pass's
-// window load, units small enough for a short queue tail (1250-neuron columns:
-// 4 units of 313; measured best on grids of 8x8, 12x12 and 24x24 columns).
-// Small networks: as many units as fit one per CU (ms per step with 108, 216,
-// 252 and 288 units of 45,000 neurons: 0.49, 0.41, 0.39 and 0.45).
-constexpr uint32_t kWindowUnitTargets = 320;
-constexpr uint32_t kWindowUnits = 256;
+// Units per column: k_collect runs one workgroup per CU, so a step takes as
+// many rounds of units as there are CUs' worth of them, each as long as a
+// unit's targets and its window loads (worth some 50 targets).  The fewest
+// target times win.  ms per 20 steps with the units per column chosen here
+// and with units of at most 320 targets: 81 columns of 1,250 neurons 13.4 (3)
+// and 14.9 (4), 100 columns 16.1 (5) and 17.1, 144 columns 23.4 (5) and 24.6,
+// 169 columns of 507 6.0 (3) and 6.5 (2); 36 columns of 1,250: 7 (252 units)
+// 7.9, 6 8.2, 8 (288) 9.1.
+constexpr uint32_t kWindowRound = 256, kWindowLoad = 50, kWindowUnitTargets = 640;
+static uint32_t window_units_per_col(uint32_t npc, uint32_t ncols) {
+  uint32_t best = 1;
+  uint64_t least = ~0ull;
+  for (uint32_t u = std::max(1u, (npc + kWindowUnitTargets - 1) / kWindowUnitTargets); u <= std::min(npc, kWindowRound); ++u) {
+    const uint64_t rounds = ((uint64_t)ncols * u + kWindowRound - 1) / kWindowRound;
+    const uint64_t cost = rounds * ((npc + u - 1) / u + kWindowLoad);
+    if (cost < least) {
+      least = cost;
+      best = u;
+    }
+  }
+  return best;
+}
 constexpr uint32_t kWindowMaxEntries = 12 * 1024;  // window entries: kWinPerThread per thread of k_collect
 
 // Block-wide work queue: the next unit for the whole workgroup (one unit
@@ -3896,11 +3911,9 @@ int dpsnn_prepare(const char *inidir, const dpsnn_options *opt, dpsnn_net **out)
       // DPSNN_WINDOW_UNITS: units wanted per step instead (tuning; results do
       // not change)
       const char *ue = getenv("DPSNN_WINDOW_UNITS");
-      const uint32_t wanted = std::max<uint32_t>((q.neuronsPerCM + kWindowUnitTargets - 1) / kWindowUnitTargets,
-                                                 kWindowUnits / std::max(q.globCFT, 1u));
-      const uint32_t unitsPerCol =
-          ue && atoi(ue) > 0 ? std::max<uint32_t>(1, ((uint32_t)atoi(ue) + q.globCFT - 1) / q.globCFT)
-                             : std::max<uint32_t>(1, wanted);
+      const uint32_t unitsPerCol = ue && atoi(ue) > 0
+                                       ? std::max<uint32_t>(1, ((uint32_t)atoi(ue) + q.globCFT - 1) / q.globCFT)
+                                       : window_units_per_col(q.neuronsPerCM, std::max(q.globCFT, 1u));
       build_window(n->par, n->con, unitsPerCol, kWindowMaxEntries, n->window, n->opt.host_threads,
                    /*fill=*/false);
     }
