@@ -1,26 +1,29 @@
 // dpsnn_engine.hip -- MI355X engine for DPSNN's per-millisecond LIFCA step.
 //
 // One network = one process's whole local network on one GPU.  Step t (one
-// reference completeTimeStep_ms, DPSNN_localNet_sim.c:22-307) is ONE kernel:
+// reference completeTimeStep_ms, DPSNN_localNet_sim.c:22-307) is:
 //
-//   k_step         per target neuron: streams the neuron's in-list (delivery
-//                  insertion order), keeps the items whose source fired in
-//                  step t-delay, orders them by arrival time (wave-wide
-//                  bucket sort in LDS on exact 64-bit keys), merges the
-//                  external bath (internal first on ties) and runs
-//                  LIFCADynamic per event in FP64, one lane per neuron.
-//                  Replaces delivery + addInputSpike +
-//                  regularDynamicTimeStep + LIFCADynamic (:837-999,
-//                  DPSNN_neuron_sim.c:289-300, :522-824).
-//                  Its tail is the fired scan of step t+1: each wave ballots
-//                  its 64 neurons' spikes into one word of the spike bitmap
-//                  of slot t+1, stores their emission times in the slot's Te
-//                  history, the last-spike ms and the per-(column, subPop)
-//                  counts, and applies STDP's LTP to the incoming synapses of
-//                  the neurons that fired.  That replaces the fired scan +
-//                  compaction + world-size-1 axonal exchange + ring insert
-//                  (:103-148, :620-806, DPSNN_spike.c:209-239) and
-//                  causalSTDP_ms (DPSNN_neuron_sim.c:94-177).
+//   k_bath         the step's external events (DPSNN_neuron_sim.c:604-640).
+//   phase 1        per target neuron, the items of its in-list (delivery
+//                  insertion order) whose source fired in step t-delay,
+//                  ordered with the bath by arrival time (wave-wide bucket
+//                  sort in LDS on exact 64-bit keys; internal first on ties):
+//                  k_gather, or for large networks k_collect + k_sort.
+//                  Replaces delivery + addInputSpike (:837-999,
+//                  DPSNN_neuron_sim.c:289-300).
+//   phase 2        LIFCADynamic per event in FP64, one lane per neuron:
+//                  k_integrate_records, k_integrate_pipe or (bath merged
+//                  here) k_integrate.  Replaces regularDynamicTimeStep +
+//                  LIFCADynamic (:522-824).  Its tail is the fired scan of
+//                  step t+1: each wave ballots its 64 neurons' spikes into
+//                  one word of the spike bitmap of slot t+1, stores their
+//                  emission times in the slot's Te history, the last-spike ms
+//                  and the per-(column, subPop) counts.  That replaces the
+//                  fired scan + compaction + world-size-1 axonal exchange +
+//                  ring insert (:103-148, :620-806, DPSNN_spike.c:209-239).
+//   k_ltp, k_stdp  STDP of a step, or of a block of steps at once
+//                  (DPSNN_neuron_sim.c:94-277).
+//   k_step         phases 1 and 2 in one launch (an option).
 //   k_compact      (only when a raster is wanted) ascending spike list of
 //                  slot t+1 appended to the device raster buffer.
 //   k_commit       (STDP, ms % 1000 == 999) the per-second weight commit.
