@@ -1183,7 +1183,8 @@ __device__ __attribute__((always_inline)) inline void integrate_records(const De
 // chain is left with the instructions that need v or c.  us per launch here
 // and in integrate_records: 1,250 and 5,000 neurons 79 and 89, 31,250 neurons
 // (489 tiles) 129 and 129, 80,000 neurons 261 and 148 (the work is more, with
-// its LDS traffic, and four workgroups fit a CU); hence kPipeTiles.
+// its LDS traffic, and four workgroups fit a CU); ms per 20 steps: 313 tiles
+// 5.54 and 5.83, 388 tiles 2.58 and 2.63, 489 tiles equal.  Hence kPipeTiles.
 typedef double f64x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) f64x2 lds_f64x2;
 typedef __attribute__((address_space(3))) float lds_f32;
@@ -1199,7 +1200,7 @@ struct PipeLds {
   uint64_t expTab[kExpTab];
 };
 constexpr int kPipeThreads = 3 * kWave;
-constexpr uint32_t kPipeTiles = 256;
+constexpr uint32_t kPipeTiles = 448;
 
 // Barrier of a pipelined tile: LDS is ordered around it, global loads in
 // flight stay in flight.
